@@ -37,6 +37,7 @@
 
 #include "bsg_device.hpp"
 #include "bsgemm.h"
+#include "pack.hpp"
 
 // The GEMM ranks the block scores itself (MODE_TOPK) when each of its waves has at most this many
 // rank items (64 blocks x 16 scores each); otherwise a separate rank launch runs first.
@@ -342,32 +343,6 @@ __global__ __launch_bounds__(256) void bsg_read_kernel(const char* __restrict__ 
     }
   }
   if ((acc.x ^ acc.y ^ acc.z ^ acc.w) == magic) sink[0] = 1u;
-}
-
-// Pack W (logical [N,K], element strides sn/sk) into the tiled K-major layout.
-// One thread per 8-element (16-byte) group of the packed slab.
-__global__ __launch_bounds__(256) void bsg_pack_kernel(const uint16_t* __restrict__ w, int64_t N,
-                                                       int64_t K, int64_t sn, int64_t skk,
-                                                       int64_t ntile, int64_t groups,
-                                                       uint16_t* __restrict__ wp) {
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= groups) return;
-  const int64_t blk = gid / (ntile * 128);
-  const int64_t rem = gid - blk * ntile * 128;
-  const int64_t t = rem >> 7;
-  const int r = (int)(rem & 127);
-  const int h = r >> 6, g = (r >> 4) & 3, c = r & 15;
-  const int64_t n = 16 * t + c;
-  const int64_t k0 = 64 * blk + 32 * h + 8 * g;
-  uint16_t v[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (n < N && k0 + e < K) ? w[n * sn + (k0 + e) * skk] : (uint16_t)0;
-  u32x4 o;
-  o.x = v[0] | ((uint32_t)v[1] << 16);
-  o.y = v[2] | ((uint32_t)v[3] << 16);
-  o.z = v[4] | ((uint32_t)v[5] << 16);
-  o.w = v[6] | ((uint32_t)v[7] << 16);
-  *(u32x4*)(wp + gid * 8) = o;
 }
 
 __global__ __launch_bounds__(256) void bsg_zero_kernel(uint32_t* __restrict__ p, int64_t n) {
@@ -986,13 +961,9 @@ int bsg_pack_weight(const void* w, int64_t N, int64_t K, int64_t stride_n, int64
   if (cdiv(K, BSG_BLOCK_K) > BSG_MAX_NBLK) return fail(BSG_ERR_UNSUPPORTED, "pack: K=%lld too large", (long long)K);
   const int64_t need = bsg_packed_bytes(N, K, dtype);
   if (wp_bytes < need) return fail(BSG_ERR_ARG, "pack: destination %lld bytes < %lld", (long long)wp_bytes, (long long)need);
-  const int64_t ntile = cdiv(N, 16);
-  const int64_t groups = cdiv(K, BSG_BLOCK_K) * ntile * 128;
-  const int64_t nb = cdiv(groups, 256);
-  if (nb > 0x7fffffff) return fail(BSG_ERR_UNSUPPORTED, "pack: too large");
-  hipLaunchKernelGGL(bsg_pack_kernel, dim3((unsigned)nb), dim3(256), 0, (hipStream_t)stream,
-                     (const uint16_t*)w, N, K, stride_n, stride_k, ntile, groups, (uint16_t*)wp);
-  hipError_t e = hipGetLastError();
+  const int rc = launch_pack(w, N, K, stride_n, stride_k, wp, stream);
+  if (rc < 0) return fail(BSG_ERR_UNSUPPORTED, "pack: too large");
+  const hipError_t e = (hipError_t)rc;
   if (e != hipSuccess) return hip_fail(e, "bsg_pack_weight launch");
   return BSG_OK;
 }
