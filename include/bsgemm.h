@@ -50,12 +50,12 @@ enum bsg_status {
 /* Launch plan of the GEMM.  A zero field means "choose automatically".
  *   split_k         : work-groups that share one output tile and split the active-block
  *                     list (fp32 partials + in-kernel deterministic reduction), >= 1
- *   cols_per_wave   : output columns per wavefront (kinds 1-4: 16, 32, 64 or 128); kinds 5-7:
+ *   cols_per_wave   : output columns per wavefront (kinds 1-4: 16, 32, 64 or 128); kinds 5-8:
  *                     the most columns one work-group may take (16 x its most subtiles)
  *   waves_per_group : wavefronts per work-group: 1, 2, 4 or 8
  *   depth           : K-blocks whose loads each wave keeps in flight: 1, 2, 4 or 8
- *   rows_per_group  : batch rows per work-group (16, 32 or 64; 1, 2, 4 or 8 for kind 3); bt
- *                     above it adds grid rows
+ *   rows_per_group  : batch rows per work-group (16, 32 or 64; 1, 2, 4 or 8 for kind 3; 128 for
+ *                     kind 8); bt above it adds row groups
  *   kind            : the kernel family.
  *     1  the waves of a work-group split its block list, each loading its own activation
  *        fragments; work-group columns = cols_per_wave.  Any split_k.
@@ -80,9 +80,14 @@ enum bsg_status {
  *        contiguous bytes per load) and read back in MFMA order instead of loaded into
  *        registers; the registers this frees allow four block-slice waves at 64 rows.
  *        split_k must be 1.
- *   Kinds 5-7 run 1-D lists only (bsg_gemm_2d rejects them), and only the tiles compiled
- *   into the library resolve (BSG_ERR_UNSUPPORTED names any other); a zero field of a kind 5-7
- *   plan takes rows 16/32/64 from bt, cols_per_wave 48, waves_per_group 4, depth 4.
+ *   Kind 8 is for batches of more than 64 rows and refused below: 128-row groups x column groups
+ *   dealt as in kind 5, both operands of every block loaded once into an LDS ring that all waves
+ *   share (waves_per_group / 2 row parts x the two channel halves); waves_per_group 8, depth (ring
+ *   stages) 4, split_k 1; no in-GEMM selection (a selection call runs a rank launch instead).
+ *   Kinds 5-8 run 1-D lists only (bsg_gemm_2d rejects them), and only the tiles compiled
+ *   into the library resolve (BSG_ERR_UNSUPPORTED names any other); a zero field of a kind 5-8
+ *   plan takes rows 16/32/64 from bt (kind 8: 128), cols_per_wave 48, waves_per_group 4 (kind 8: 8),
+ *   depth 4.
  * kind 0 here resolves by heuristic to kind 1 (bt <= 16) or kind 2 (larger bt).  The Python
  * layer does not rely on it: its plans come from a table tuned on the MI355X
  * (bsa_mi355x/tuned_plans.json) whose entries name kinds 1, 2, 4, 5, 6 and 7, or from

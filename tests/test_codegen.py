@@ -8,6 +8,9 @@ that no result test can pin reliably (CPU only: hipcc cross-compiles the device 
 - Kinds 5/6 keep their main loops free of full pipeline drains (`s_waitcnt vmcnt(0)` inside a
   loop that runs MFMAs) except in the four tiles where the register allocator is known to force
   one; unrelated edits to the shared device code have added drains to other tiles before.
+- Kind 8 waits for a ring stage by the count of loads every wave issues per slot, so between two
+  barriers of its pipeline each wave must issue exactly that many, whatever its lanes' bounds (a
+  branch around a load would change the count), and must not wait for all of them.
 """
 from __future__ import annotations
 
@@ -89,3 +92,25 @@ def test_variable_width_kernels_keep_their_loops_free_of_drains(tmp_path):
             btt, nsub, wb, depth, kh = [int(a) for a in re.findall(r"Li(\d+)E", name)][:5]
             assert kh == 1 and (btt, nsub, wb, depth) in known, name
     assert names >= 100
+
+
+def test_rows_kernel_issues_whole_stages_between_barriers(tmp_path):
+    asm = _device_asm("tiles_k8.hip", tmp_path)
+    checked = 0
+    for name, body in _functions(asm, "_ZN12_GLOBAL__N_120bsg_gemm_rows_kernel"):
+        btt, nsub, rw, depth = [int(a) for a in re.findall(r"Li(\d+)E", name)][:4]
+        waves = 2 * rw
+        per_slot = 2 * btt // waves + -(-2 * nsub // waves)
+        lds = [k for k, line in enumerate(body) if "buffer_load_dwordx4" in line and " lds" in line]
+        pipe = body[lds[0]:lds[-1] + 1]
+        # the prologue fills the ring, then every slot (the loop holds `depth` of them) refills one stage
+        parts = "\n".join(pipe).split("s_barrier")
+        counts = [sum("buffer_load_dwordx4" in x for x in part.split("\n")) for part in parts]
+        assert sum(counts) == len(lds) == 2 * depth * per_slot, (name, counts)
+        assert counts[0] == depth * per_slot and counts[1] == 0 and counts[2:] == [per_slot] * depth, (name, counts)
+        assert not any("vmcnt(0)" in x for x in pipe), name
+        # the only branch inside the pipeline is the loop's back edge
+        labels = [x for x in pipe if re.match(r"^\.LBB\d+_\d+:", x.strip())]
+        assert len(labels) <= 1 and not any("s_cbranch_exec" in x for x in pipe), name
+        checked += 1
+    assert checked == 8

@@ -347,3 +347,14 @@ def test_bench_kernel_shares_weight_points_by_launches_per_step():
     assert k1["points"] == ["a", "c"] and abs(k1["time_share"] - 60 / 110) < 1e-4
     assert abs(k1["GBps"] - 28_000_000 / 60e-6 / 1e9) < 0.1
     assert abs(out["bsg_gemm_vt_kernel"]["frac"] - (20_000_000 / 50e-6 / 1e9) / bench.HBM_PEAK_GBS) < 1e-4
+
+
+def test_many_rows_plans_resolve_unchanged():
+    """Every plan tuning.many_rows_plan gives past 64 rows names a compiled tile that the library
+    takes as it is, whatever the width, and its tile covers the batch."""
+    for bt in (65, 72, 96, 127, 128, 129, 192, 255, 256, 257, 300, 512, 700, 1024, 5000):
+        for n in (1, 16, 100, 1000, 2048, 4096, 4097, 5120, 6912, 8192, 11008, 12288, 13827, 16384, 22016, 32000):
+            p = tuning.many_rows_plan(bt, n)
+            q = bsa.Plan(*p.as_tuple())
+            assert bsa.load().bsg_plan_resolve(bt, n, 64, 31, 256, ctypes.byref(q)) == 0, (bt, n, p.as_tuple())
+            assert q.as_tuple() == p.as_tuple() and p.rows_per_group >= 64

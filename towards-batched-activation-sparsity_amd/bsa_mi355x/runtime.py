@@ -212,13 +212,15 @@ def resolve_plan(bt: int, n: int, nblk: int, na: int, device: torch.device, plan
                  dense: bool = False, lookup_plan: bool = True, select: bool = False) -> Plan:
     """Resolve a (partial) plan for a problem.  With no plan (or an all-zero one) the tuned
     table (tuning.lookup; select=True: the entries timed as selection + GEMM first) is consulted
-    first; remaining zero fields are filled by the library's heuristics; tile fields that name a
+    first (past 64 rows, tuning.many_rows_plan); remaining zero fields are filled by the library's heuristics; tile fields that name a
     kernel that is not instantiated fall back to automatic (the split-K factor is kept)."""
     lib = load()
     if lookup_plan and (plan is None or not any(plan.as_tuple())):
         from . import tuning
 
         tuned = tuning.lookup(bt, n, nblk, na, dense=dense, select=select)
+        if tuned is None and bt > 64:
+            tuned = tuning.many_rows_plan(bt, n)
         if tuned is not None:
             plan = tuned
     req = plan.as_tuple() if plan is not None else (0, 0, 0, 0, 0, 0)
@@ -705,8 +707,8 @@ def dense_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, cache_p
 def kernel_tiles() -> Sequence[tuple]:
     """Instantiated (kind, rows_per_group, cols_per_wave, waves_per_group, depth) tuples."""
     out = []
-    for kind in (1, 2, 3, 4, 5, 6, 7):
-        for rows in ((1, 2, 4, 8) if kind == 3 else (16, 32, 64)):
+    for kind in (1, 2, 3, 4, 5, 6, 7, 8):
+        for rows in ((1, 2, 4, 8) if kind == 3 else (128,) if kind == 8 else (16, 32, 64)):
             for cols in ((16, 32, 48, 64, 96) if kind >= 5 else (16, 32, 64, 128)):
                 for waves in (1, 2, 4, 8):
                     for depth in (1, 2, 4, 8):

@@ -43,6 +43,28 @@ def rows_bucket(bt: int) -> int:
     return 16 if bt <= 16 else (32 if bt <= 32 else 64)
 
 
+# Compute units the launch plans are made for.
+_CUS = 256
+
+
+def many_rows_plan(bt: int, n: int) -> Plan:
+    """Plan for more than 64 rows, by size.  What a compute unit takes in per K-block, (rows +
+    columns of its tile) x 128 bytes, bounds these launches.  Where 128-row groups leave at least
+    3 column subtiles to each compute unit, kind 8 takes them (N = 11008, 31 blocks: 256 rows 23.2
+    us against 43.6 with four 64-row groups, 128 rows 18.4 / 23.0, 72 rows 15.2 / 19.3; N = 22016,
+    128 rows 25.7 / 36.8).  Below that the tile is nearer square with 64 rows: kind 7 up to 3
+    subtiles (N = 4096, 128 rows: 9.8, kind 8 12.9), and past 3 the 128-column tile of kind 4 with
+    the list split in two (N = 4096, 256 rows: 31 blocks 14.5, 83 blocks 27.1; kind 8 14.7, 31.4)."""
+    tiles = -(-int(n) // 16)
+    s128 = -(-tiles * -(-int(bt) // 128) // _CUS)
+    if s128 >= 3:
+        return Plan(1, 48 if s128 == 3 else 64 if s128 == 4 else 96, 8, 4, 128, 8)
+    s64 = -(-tiles * -(-int(bt) // 64) // _CUS)
+    if s64 <= 3:
+        return Plan(1, 32 if s64 <= 2 else 48, 4, 2, 64, 7)
+    return Plan(2, 32, 8, 4, 64, 4)
+
+
 # ---------------------------------------------------------------------------------------
 # Run-time lookup
 
@@ -69,7 +91,8 @@ def load_table(path: str = TABLE_PATH) -> List[dict]:
 
 def lookup(bt: int, n: int, nblk: int, na: int, dense: bool = False, select: bool = False) -> Optional[Plan]:
     """Best tabulated plan for (bt, N, nblk, na): same N and block count, same 16/32/64-row
-    bucket, nearest batch, then the dense entry (dense=True) or the nearest active-block count.
+    bucket, nearest batch, then the dense entry (dense=True) or the nearest active-block count;
+    past 64 rows, the batches the table was tuned for, many_rows_plan.
     select=True (a selection + GEMM, whose GEMM ranks the block scores itself) prefers the
     entries timed that way (refine_select) and falls back to the plain GEMM's.  None when the
     shape is not tabulated."""
@@ -88,6 +111,8 @@ def _lookup(bt: int, n: int, nblk: int, na: int, dense: bool, select: bool) -> O
     cands = _INDEX.get((n, nblk))
     if not cands:
         return None
+    if bt > 64:
+        return many_rows_plan(bt, n)
     rb = rows_bucket(bt)
     same = [e for e in cands if rows_bucket(int(e["bt"])) == rb]
     if select and not dense:
@@ -184,8 +209,9 @@ def candidate_plans(bt: int, na: int, nblk: int) -> List[Plan]:
                 out.append(Plan(1, cols, waves, depth, rows, kind))
             continue
         if kind >= 5:  # variable-width column groups: the chip is filled without split-K
-            # 32- and 64-row batches also try two row groups of half the rows (as below)
-            if rows == rb or (rb >= 32 and rows == rb // 2):
+            # 32- and 64-row batches also try two row groups of half the rows (as below), larger
+            # ones the 128-row groups of kind 8
+            if rows == rb or (rows == 128 and bt > 64) or (rb >= 32 and rows == rb // 2):
                 out.append(Plan(1, cols, waves, depth, rows, kind))
             continue
         # 32-row batches also try 64-row tiles; 32- and 64-row batches also try two row groups of

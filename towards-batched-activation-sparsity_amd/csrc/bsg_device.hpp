@@ -48,7 +48,7 @@ struct GemmParams {
 
 typedef void (*GemmFn)(GemmParams);
 
-enum { KIND_KSPLIT = 1, KIND_XLDS = 2, KIND_FMA = 3, KIND_XLDS_KH = 4, KIND_VT = 5, KIND_VT1 = 6, KIND_VT1X = 7 };
+enum { KIND_KSPLIT = 1, KIND_XLDS = 2, KIND_FMA = 3, KIND_XLDS_KH = 4, KIND_VT = 5, KIND_VT1 = 6, KIND_VT1X = 7, KIND_ROWS = 8 };
 
 // 1-D and, for tiles of at most 64 columns per work-group, 2-D (active output blocks) entries.
 // f16_sel: the fp16 1-D form compiled with the in-GEMM top-k (MODE_TOPK; on 16-row tiles also
@@ -65,7 +65,7 @@ struct TileTable {
   int n;
 };
 
-extern const TileTable kTilesK1R16, kTilesK1R32, kTilesK1R64, kTilesK2, kTilesK4, kTilesK3, kTilesK5, kTilesK7;
+extern const TileTable kTilesK1R16, kTilesK1R32, kTilesK1R64, kTilesK2, kTilesK4, kTilesK3, kTilesK5, kTilesK7, kTilesK8;
 
 }  // namespace bsgk
 

@@ -463,7 +463,7 @@ __global__ __launch_bounds__(1024) void bsg_nmask_kernel(const uint8_t* __restri
 
 // The whole instantiated tile set, one table per translation unit.
 const TileTable* const kTables[] = {&kTilesK1R16, &kTilesK1R32, &kTilesK1R64, &kTilesK2, &kTilesK4, &kTilesK3,
-                                    &kTilesK5, &kTilesK7};
+                                    &kTilesK5, &kTilesK7, &kTilesK8};
 
 const KernelEntry* find_kernel_scan(int kind, int rows, int nsub, int wpg, int depth) {
   for (const TileTable* t : kTables)
@@ -541,16 +541,17 @@ int resolve_fma(int64_t bt, int32_t na, bsg_plan* pl) {
   return BSG_OK;
 }
 
-// Kind 5, 6 and 7 plans: explicit or tuned only; no split-K (their groups already fill the chip).
+// Kind 5 to 8 plans: explicit or tuned only; no split-K (their groups already fill the chip).
 int resolve_vt(bsg_plan* pl) {
   const int rpg = pl->rows_per_group;
-  if (rpg != 16 && rpg != 32 && rpg != 64)
-    return fail(BSG_ERR_UNSUPPORTED, "plan: kind %d rows_per_group=%d (16, 32 or 64)", pl->kind, rpg);
+  if (pl->kind == KIND_ROWS ? rpg != 128 : (rpg != 16 && rpg != 32 && rpg != 64))
+    return fail(BSG_ERR_UNSUPPORTED, "plan: kind %d rows_per_group=%d (%s)", pl->kind, rpg,
+                pl->kind == KIND_ROWS ? "128" : "16, 32 or 64");
   if (pl->split_k == 0) pl->split_k = 1;
   if (pl->split_k != 1)
     return fail(BSG_ERR_UNSUPPORTED, "plan: kind %d needs split_k=1 (got %d)", pl->kind, pl->split_k);
   if (pl->cols_per_wave == 0) pl->cols_per_wave = 48;
-  if (pl->waves_per_group == 0) pl->waves_per_group = 4;
+  if (pl->waves_per_group == 0) pl->waves_per_group = pl->kind == KIND_ROWS ? 8 : 4;
   if (pl->depth == 0) pl->depth = 4;
   if (pl->cols_per_wave % 16 != 0 ||
       !find_kernel(pl->kind, rpg, pl->cols_per_wave / 16, pl->waves_per_group, pl->depth))
@@ -574,12 +575,15 @@ int resolve(int64_t bt, int64_t N, int32_t nblk, int32_t na, int32_t cu, bsg_pla
   if (bt <= 0 || N <= 0 || nblk <= 0 || na < 0 || cu <= 0)
     return fail(BSG_ERR_ARG, "plan: bt=%lld N=%lld nblk=%d na=%d cu=%d", (long long)bt, (long long)N,
                 nblk, na, cu);
-  if (pl->kind < 0 || pl->kind > KIND_VT1X)
+  if (pl->kind < 0 || pl->kind > KIND_ROWS)
     return fail(BSG_ERR_UNSUPPORTED, "plan: kind=%d (1 = waves split the block list, 2 = X tile in LDS, "
                 "3 = fp32 dot products for 1-8 rows, 4 = as 2 with channel-half waves, 5 = variable-width "
                 "column groups, 6 = as 5 with waves splitting blocks only, 7 = as 6 with the activations "
-                "loaded into LDS)", pl->kind);
-  if (pl->kind == KIND_VT || pl->kind == KIND_VT1 || pl->kind == KIND_VT1X) {
+                "loaded into LDS, 8 = 128-row groups)", pl->kind);
+  if (pl->kind >= KIND_VT) {
+    if (pl->kind == KIND_ROWS && bt <= 64)
+      return fail(BSG_ERR_UNSUPPORTED, "plan: kind 8 is for more than 64 rows (bt=%lld)", (long long)bt);
+    if (pl->rows_per_group == 0 && pl->kind == KIND_ROWS) pl->rows_per_group = 128;
     if (pl->rows_per_group == 0) pl->rows_per_group = bt <= 16 ? 16 : (bt <= 32 ? 32 : 64);
     return resolve_vt(pl);
   }
@@ -824,9 +828,9 @@ int launch_gemm(int mode, const void* x, int64_t ldx, int64_t bt, int64_t K, con
                 "cols_per_wave x column waves)", (long long)gc);
   // 2-D: 64 / gc tiles per active output block (a device-side count leaves tiles idle)
   const int64_t ygroups = cdiv(bt, pl.rows_per_group);
-  const bool vt = pl.kind == KIND_VT || pl.kind == KIND_VT1 || pl.kind == KIND_VT1X;
+  const bool vt = pl.kind >= KIND_VT;
   if (vt && ex.nidx != nullptr)
-    return fail(BSG_ERR_UNSUPPORTED, "2-D: kinds 5-7 (variable-width column groups) have no 2-D form");
+    return fail(BSG_ERR_UNSUPPORTED, "2-D: kinds 5-8 (variable-width column groups) have no 2-D form");
   const int64_t n_tiles = vt ? vt_groups(N, ygroups, device_cu_count(), &pl)
                           : ex.nidx != nullptr ? (int64_t)ex.nn * (64 / gc) : cdiv(npad, gc);
   if (n_tiles * pl.split_k > 0x7fffffff || ygroups > 65535) return fail(BSG_ERR_UNSUPPORTED, "grid too large");
@@ -869,6 +873,10 @@ int launch_gemm(int mode, const void* x, int64_t ldx, int64_t bt, int64_t K, con
   p.tl = timeline_slot((int64_t)n_tiles * pl.split_k * ygroups);
 
   dim3 grid((unsigned)(n_tiles * pl.split_k), (unsigned)ygroups, 1);
+  if (pl.kind == KIND_ROWS) {  // row groups are folded into the x axis (see the kernel)
+    if (n_tiles * ygroups > 0x7fffffff) return fail(BSG_ERR_UNSUPPORTED, "grid too large");
+    grid = dim3((unsigned)(n_tiles * ygroups), 1, 1);
+  }
   dim3 block((unsigned)(64 * pl.waves_per_group), 1, 1);
   const bool topk = mode == MODE_TOPK || mode == MODE_TOPK_SELF;
   GemmFn fn = topk ? (dtype == BSG_F16 ? ke->f16_sel : nullptr)
