@@ -204,6 +204,19 @@ int bsg_gemm_2d(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* w
                 void* y, int64_t ldy, int dtype,
                 void* ws, int64_t ws_bytes, const bsg_plan* plan, void* stream);
 
+/* bsg_gemm_2d with its lists sorted ascending by the GEMM itself (no sort launch), as the
+ * reference's entry does first (sort_active_k_blocks, sort_active_n_blocks; KRN:3498-3850).
+ *   sort_active  : non-zero sorts the K-block list while it is staged (num_active <= BSG_MAX_NBLK / 2)
+ *   n_sorted_out : non-null (device, room for num_n) when n_blocks holds num_n_list ids in any order
+ *                  (at most 512, else BSG_ERR_UNSUPPORTED): the num_n lowest are computed and
+ *                  written there ascending; null takes n_blocks[num_n] as it is.
+ * With num_n = 0 nothing is written.  The result is bsg_gemm_2d on the sorted lists, bit for bit. */
+int bsg_gemm_2d_sorted(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
+                       const int32_t* active_blocks, int32_t num_active, int sort_active,
+                       const int32_t* n_blocks, int32_t num_n_list, int32_t num_n, int32_t* n_sorted_out,
+                       int compact, void* y, int64_t ldy, int dtype,
+                       void* ws, int64_t ws_bytes, const bsg_plan* plan, void* stream);
+
 /* Scatter a compact 2-D output back to the dense N axis:
  * out[r, 64 n_blocks[i] + c] = compact[r, 64 i + c] for c < 64 and 64 n_blocks[i] + c < N,
  * i < num_n (or *num_n_dev when set); other columns of out are untouched.  16-bit elements.

@@ -246,3 +246,57 @@ def test_2d_split_k_workspace_reuse_across_block_counts(dev):
         assert pl.split_k == 4
         torch.cuda.synchronize()
         _check(y.float().cpu().numpy(), x, w_nk, kb, nb, False, f"workspace reuse nn={nn}")
+
+
+@pytest.mark.parametrize("plan", [None, (1, 16, 4, 4, 16, 1), (3, 32, 2, 4, 16, 1), (2, 16, 4, 4, 32, 2),
+                                  (1, 16, 8, 4, 64, 4), (1, 16, 4, 4, 8, 3)])
+@pytest.mark.parametrize("nl,nn,na", [(2, 2, 2), (3, 1, 9), (64, 17, 63), (130, 130, 64), (512, 300, 40)])
+def test_2d_lists_sorted_in_the_kernel(dev, plan, nl, nn, na):
+    """Unsorted lists, with equal and out-of-range ids among them: the same bits as the call on the
+    sorted lists, and the sorted output list; in place and compact."""
+    kdim, n = 4096, 64 * 300 - 40
+    bt = plan[4] if plan else 7
+    rng = np.random.default_rng(nl + na)
+    x, w_nk, _ = case(91, bt, kdim, n, 1, "normal")
+    xt, packed = to_dev(x, dev), bsa.pack_weight(to_dev(w_nk, dev))
+    kb = rng.permutation(64)[:na].astype(np.int32)
+    kb[-1] = kb[0] if na > 2 else kb[-1]  # an id twice
+    nb = np.r_[rng.permutation(300), rng.integers(0, 300, 212)][:nl].astype(np.int32)
+    if nl > 2:
+        nb[nl // 2] = 300 + nl  # no such block: sorts last
+        nb[0] = -1              # nor this one: sorts first
+    p = bsa.Plan(*plan) if plan else None
+    for compact in (False, True):
+        got = torch.full((bt, nn * 64 if compact else n), SENTINEL, dtype=torch.float16, device=dev)
+        want = got.clone()
+        ids = torch.full((nn,), -7, dtype=torch.int32, device=dev)
+        print(f"2-D sorted plan={plan} nl={nl} nn={nn} na={na} compact={compact}", flush=True)
+        s2d.gemm_2d_packed(xt, packed, n, to_dev(kb, dev), to_dev(nb, dev), got, num_n=nn, compact=compact, plan=p,
+                           sort_active=True, n_sorted_out=ids)
+        s2d.gemm_2d_packed(xt, packed, n, to_dev(np.sort(kb), dev), to_dev(np.sort(nb)[:nn].copy(), dev), want,
+                           compact=compact, plan=p)
+        assert np.array_equal(ids.cpu().numpy(), np.sort(nb)[:nn])
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_2d_entry_points_past_the_in_kernel_sort(dev):
+    """Lists longer than the kernels sort themselves (1024 K-blocks, 512 output blocks) go through a
+    sort launch; an empty output limit returns the sorted list."""
+    kdim, n = 64 * 1100, 64 * 520
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(2, 1, kdim, generator=g, device=dev).half()
+    w = (torch.randn(n, kdim, generator=g, device=dev) * 0.02).half()
+    for na, nn in ((1030, 515), (1030, 3), (5, 515)):
+        kb = torch.randperm(1100, generator=g, device=dev)[:na].int()
+        nb = torch.randperm(520, generator=g, device=dev)[:nn].int()
+        out = torch.zeros(2, 1, n, dtype=torch.float16, device=dev)
+        _, blocks = s2d._prepacked_block_sparse_gemm_2d_from_active_blocks(x, w, kb, nb, out, cache_prefix="long2d")
+        assert torch.equal(blocks, nb.sort()[0])
+        ch = (kb.long()[:, None] * 64 + torch.arange(64, device=dev)).reshape(-1)
+        co = (nb.long()[:, None] * 64 + torch.arange(64, device=dev)).reshape(-1)
+        ref = x.view(2, -1)[:, ch].float() @ w[co][:, ch].float().t()
+        got = out.view(2, n)[:, co].float()
+        assert ((got - ref).norm() / ref.norm()).item() < 1e-3
+    _, blocks = s2d._prepacked_block_sparse_gemm_2d_from_active_blocks(x, w, kb, nb[:9], out, active_n_blocks_limit=0,
+                                                                       cache_prefix="long2d")
+    assert torch.equal(blocks, nb[:9].sort()[0]) and not torch.any(out)

@@ -21,6 +21,7 @@ from ._lib import Plan, check, load
 from .runtime import (BLOCK_K, MAX_NBLK, _cu_count, _dtype_code, _pad_k, _packed_entry, _require_cuda,
                       _sort_active_blocks_asc, _stream_handle, _workspace, ctypes_byref, resolve_plan)
 
+SORT_N_MAX = 512  # output-block list entries that the GEMM sorts itself (bsg_gemm_2d_sorted)
 INDEX_BLOCK_OUT_META_SIZE = 64  # output-block width of the 2-D path (KRN:19)
 BLOCK_N_OUT = INDEX_BLOCK_OUT_META_SIZE
 
@@ -85,13 +86,17 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
                    n_blocks: torch.Tensor, y2d: torch.Tensor, *, num_active: Optional[int] = None,
                    num_active_dev: Optional[torch.Tensor] = None, num_n: Optional[int] = None,
                    num_n_dev: Optional[torch.Tensor] = None, compact: bool = False, plan: Optional[Plan] = None,
-                   workspace_prefix: str = "gemm2d") -> Plan:
+                   workspace_prefix: str = "gemm2d", sort_active: bool = False,
+                   n_sorted_out: Optional[torch.Tensor] = None) -> Plan:
     """One 2-D block-sparse GEMM on packed weights (bsg_gemm_2d).
 
     x2d [bt, K]; `active_blocks` int32 K-block list (None: every K-block) with optional host
     length `num_active` and device count `num_active_dev`; `n_blocks` int32 list of active
     64-column output blocks (ascending), host length `num_n`, optional device count
-    `num_n_dev`.  compact=False: y2d is [bt, N] and only the active blocks' columns are
+    `num_n_dev`.  sort_active: the GEMM sorts the K-block list ascending itself (at most
+    MAX_NBLK // 2 entries); n_sorted_out (int32, at least num_n): n_blocks is in any order (at most
+    SORT_N_MAX entries) and the GEMM takes its num_n lowest, writing them there ascending (both
+    with host counts only).  compact=False: y2d is [bt, N] and only the active blocks' columns are
     written; compact=True: y2d is [bt, num_n * 64], list entry i at columns 64i.."""
     lib = load()
     dev = _require_cuda(x2d, packed, y2d)
@@ -110,7 +115,14 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
         raise ValueError(f"y must be [bt, {width}] with unit column stride, got {tuple(y2d.shape)}")
     if bt == 0 or nn == 0:
         return Plan()
+    sort = sort_active or n_sorted_out is not None
+    if sort and (num_active_dev is not None or num_n_dev is not None):
+        raise ValueError("in-kernel sorting takes host counts")
     nb = _int32_dev(n_blocks, dev)
+    if n_sorted_out is not None and (n_sorted_out.dtype != torch.int32 or n_sorted_out.device != dev
+                                     or not n_sorted_out.is_contiguous() or int(n_sorted_out.numel()) < nn
+                                     or n_sorted_out.data_ptr() == nb.data_ptr()):
+        raise ValueError(f"n_sorted_out must be another int32 tensor of at least {nn} entries on {dev}")
     if active_blocks is not None:
         ab = _int32_dev(active_blocks, dev)
         na = int(ab.numel() if num_active is None else num_active)
@@ -123,6 +135,14 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
     ws_ptr = (_workspace(workspace_prefix, dev, ws_bytes, (bt, n_dim) + pl.as_tuple()).data_ptr()
               if ws_bytes > 0 else None)
     with torch.cuda.device(dev):
+        if sort:
+            check(lib.bsg_gemm_2d_sorted(
+                x2d.data_ptr(), x2d.stride(0), bt, x2d.shape[1], packed.data_ptr(), n_dim,
+                ab.data_ptr() if ab is not None and na > 0 else None, na if ab is not None else 0,
+                1 if sort_active else 0, nb.data_ptr(), int(nb.numel()), nn,
+                n_sorted_out.data_ptr() if n_sorted_out is not None else None, 1 if compact else 0, y2d.data_ptr(),
+                y2d.stride(0), code, ws_ptr, ws_bytes, ctypes_byref(pl), _stream_handle(dev)))
+            return pl
         rc = lib.bsg_gemm_2d(x2d.data_ptr(), x2d.stride(0), bt, x2d.shape[1], packed.data_ptr(), n_dim,
                              ab.data_ptr() if ab is not None and na > 0 else None, na if ab is not None else 0,
                              num_active_dev.data_ptr() if num_active_dev is not None else None,
@@ -237,27 +257,32 @@ def _prepacked_block_sparse_gemm_2d_from_active_blocks(
         return None, torch.empty((0,), device=dev, dtype=torch.int32)
     entry = _packed_entry(weight, BLOCK_K, cache_prefix)
     kb = _int32_dev(active_k_blocks, dev)[:num_k].contiguous()
-    if sort_active_k_blocks:
+    # the GEMM sorts both lists itself, up to the entries its staging holds
+    bt = bsz * seqlen
+    sort_k = sort_active_k_blocks and 1 < num_k <= MAX_NBLK // 2
+    if sort_active_k_blocks and not sort_k:
         kb = _sort_active_blocks_asc(kb)
     if active_n_blocks is None and active_n_mask_u8 is not None:
         active_n_blocks = _get_cached_active_n_blocks_delta(active_n_mask_u8, f"{cache_prefix}_nout", BLOCK_N_OUT)
     if active_n_blocks is None:
         active_n_blocks = torch.arange((n_dim + BLOCK_N_OUT - 1) // BLOCK_N_OUT, device=dev, dtype=torch.int32)
     nb = _int32_dev(active_n_blocks, dev)
-    if sort_active_n_blocks:
+    sort_n = sort_active_n_blocks and bt > 0 and 1 < int(nb.numel()) <= SORT_N_MAX
+    if sort_active_n_blocks and not sort_n:
         nb = _sort_active_blocks_asc(nb)
     num_n = int(nb.numel()) if active_n_blocks_limit is None else min(int(active_n_blocks_limit), int(nb.numel()))
     if num_n <= 0:
         out.zero_()
-        return None, nb
-    nb_ret = nb[:num_n].contiguous()
-    bt = bsz * seqlen
+        return None, _sort_active_blocks_asc(nb) if sort_n else nb
+    nb_ret = torch.empty(num_n, dtype=torch.int32, device=dev) if sort_n else nb[:num_n].contiguous()
+    lists = {"num_n": num_n, "sort_active": sort_k, "n_sorted_out": nb_ret if sort_n else None}
+    nb_in = nb if sort_n else nb_ret
     x2d = x.reshape(bt, m_dim)
     if compact_output:
         width = num_n * BLOCK_N_OUT
         y_c = _temp_buffer(f"{cache_prefix}_compact2d_out", (bt, width), x.dtype, dev)
-        gemm_2d_packed(x2d, entry.packed, n_dim, kb, nb_ret, y_c, compact=True,
-                       workspace_prefix=f"{cache_prefix}_ws2d")
+        gemm_2d_packed(x2d, entry.packed, n_dim, kb, nb_in, y_c, compact=True,
+                       workspace_prefix=f"{cache_prefix}_ws2d", **lists)
         y_c3 = y_c.view(bsz, seqlen, width)
         if scatter_compact_to_dense:
             if zero_fill_out:
@@ -268,7 +293,8 @@ def _prepacked_block_sparse_gemm_2d_from_active_blocks(
         raise ValueError(f"out must be a contiguous [B, S, N={n_dim}], got {tuple(out.shape)}")
     if zero_fill_out:
         out.zero_()
-    gemm_2d_packed(x2d, entry.packed, n_dim, kb, nb_ret, out.view(bt, n_dim), workspace_prefix=f"{cache_prefix}_ws2d")
+    gemm_2d_packed(x2d, entry.packed, n_dim, kb, nb_in, out.view(bt, n_dim), workspace_prefix=f"{cache_prefix}_ws2d",
+                   **lists)
     return None, nb_ret
 
 

@@ -35,6 +35,9 @@ struct GemmParams {
   int32_t keyed;
   // MODE_LIST: sort the list ascending while staging it (at most BSG_MAX_NBLK / 2 entries)
   int32_t sort_list;
+  // The 2-D forms, which have no top-k modes, take an unsorted output-block list through the same
+  // fields: idx_out set means that nidx holds `keyed` ids in any order (at most BSG_2D_SORT_MAX),
+  // that the kernel takes the nn lowest, and that work-group (0, 0) writes them ascending to idx_out.
   // 2-D sparsity: ascending active 64-column output blocks (null: every column), their count
   // (host value, or the device one when nn_dev is set), whether Y is compact (active blocks
   // side by side), and the width Y stores are bounded by (N, or nn * 64 when compact)
@@ -133,6 +136,9 @@ enum { MODE_LIST = 0, MODE_BITMAP = 1, MODE_DENSE = 2, MODE_TOPK = 3, MODE_TOPK_
 // block-list buffer, and a one-wave work-group flags at most 8 per thread.
 #define BSG_TOPK_MAX_NBLK 512
 #define BSG_SELF_MAX_ROWS 8
+
+// The 2-D kernels sort an output-block list of up to this many entries themselves.
+#define BSG_2D_SORT_MAX 512
 
 // Kind 3 activation staging: 1 KiB loads per wave, and the LDS it may take.
 #define BSG_FMA_X_LOADS 16
@@ -398,6 +404,72 @@ __device__ __forceinline__ void tile_of_group(int split_k, int* tile, int* sk) {
   *sk = lid - *tile * split_k;
 }
 
+// Distinct ids of [0, universe) (at most BSG_MAX_NBLK) in ascending order, handed to emit(position,
+// id): the ids set bits of an LDS bitmap, and each set bit's position is the count of set bits below
+// it.  `first` is ids[threadIdx.x], loaded by the caller ahead of whatever it waits for.  Returns
+// false, before any emit, when an id is out of range or occurs twice.  s_bm holds BSG_MAX_NBLK / 32
+// words that emit does not touch; the emitted values are unfenced.  Three dependent LDS steps whatever
+// the length, where ranking every entry against the list takes one LDS read per entry: a q/k/v/o
+// launch at 2 rows on 13 unsorted entries 4.58 -> 4.19 us, down at 16 rows on 86 entries (an eager
+// call) 14.3 -> 12.1.
+template <int NT, typename Emit>
+__device__ __forceinline__ bool sort_by_bitmap(const int32_t* ids, int n, int universe, int first, uint32_t* s_bm,
+                                               Emit emit) {
+  const int tid = threadIdx.x;
+  if (tid < BSG_MAX_NBLK / 32) s_bm[tid] = 0;
+  __syncthreads();
+  int odd = 0;
+  for (int i = tid; i < n; i += NT) {
+    const int id = i == tid ? first : ids[i];
+    const uint32_t bit = 1u << (id & 31);
+    odd |= (unsigned)id >= (unsigned)universe || (atomicOr(&s_bm[id >> 5], bit) & bit) != 0;
+  }
+  if (__syncthreads_or(odd)) return false;
+  for (int t = tid; t < universe; t += NT) {
+    const uint32_t w = s_bm[t >> 5], bit = 1u << (t & 31);
+    if (w & bit) {
+      int r = __popc(w & (bit - 1));
+      for (int k = 0; k < (t >> 5); ++k) r += __popc(s_bm[k]);
+      emit(r, t);
+    }
+  }
+  return true;
+}
+
+// The bi-th lowest id of an unsorted output-block list, found by every work-group for itself (a
+// down call at 16 rows on 86 K-blocks and 32 output blocks: 11.1 us, 13.4 with both lists ranked
+// entry by entry, 39.5 with two sort launches in front): a bitmap of the ids, or, for a list with
+// equal or out-of-range ids, each entry ranked against the whole list (equal ids by position).
+template <int NT>
+__device__ __forceinline__ int nth_output_block(const GemmParams& p, int bi) {
+  __shared__ int s_nk[BSG_2D_SORT_MAX];
+  __shared__ int s_nth;
+  const int tid = threadIdx.x, nl = p.keyed;
+  const bool publish = blockIdx.x == 0 && blockIdx.y == 0;
+  auto emit = [&](int r, int id) {
+    if (r == bi) s_nth = id;
+    if (publish && r < p.nn) p.idx_out[r] = id;
+  };
+  const int nb = (p.N + 63) / 64;
+  if (!sort_by_bitmap<NT>(p.nidx, nl, nb < BSG_MAX_NBLK ? nb : BSG_MAX_NBLK, tid < nl ? p.nidx[tid] : 0,
+                          (uint32_t*)s_nk, emit)) {
+    for (int i = tid; i < nl; i += NT) s_nk[i] = p.nidx[i];
+    __syncthreads();
+    for (int i = tid; i < nl; i += NT) {
+      const int ki = s_nk[i];
+      int r = 0;
+#pragma unroll 8
+      for (int j = 0; j < nl; ++j) {
+        const int kj = s_nk[j];
+        r += (kj < ki) | ((kj == ki) & (j < i));
+      }
+      emit(r, ki);
+    }
+  }
+  __syncthreads();
+  return s_nth;
+}
+
 // Columns of column tile `tile` (gc columns wide): n0 = first weight column it reads, n0y =
 // first output column it writes.  N2D (2-D sparsity, a separate instantiation so the 1-D
 // kernels carry none of it): tile t is piece t % (64/gc) of active 64-column block
@@ -405,26 +477,27 @@ __device__ __forceinline__ void tile_of_group(int split_k, int* tile, int* sk) {
 // the tile has no block (past the device-side count): the whole work-group then returns
 // before any barrier.  A block id outside [0, ceil(N/64)) reads past the packed columns (zero
 // weights) and writes nothing.
-template <bool N2D>
+template <bool N2D, int NT>
 __device__ __forceinline__ bool tile_columns(const GemmParams& p, int tile, int gc, int* n0, int* n0y) {
   if constexpr (!N2D) {
     *n0 = *n0y = tile * gc;
     return true;
+  } else {
+    const int per = 64 / gc;
+    const int bi = tile / per;
+    int nn = p.nn;
+    if (p.nn_dev != nullptr) {
+      const int d = __builtin_amdgcn_readfirstlane(*p.nn_dev);
+      nn = d < 0 ? 0 : (d < nn ? d : nn);
+    }
+    if (bi >= nn) return false;
+    const int off = (tile - bi * per) * gc;
+    const int nb = __builtin_amdgcn_readfirstlane(p.idx_out != nullptr ? nth_output_block<NT>(p, bi) : p.nidx[bi]);
+    const bool ok = nb >= 0 && nb < (p.N + 63) / 64;
+    *n0 = ok ? nb * 64 + off : p.npad;
+    *n0y = p.ncompact ? bi * 64 + off : (ok ? *n0 : p.ny);
+    return true;
   }
-  const int per = 64 / gc;
-  const int bi = tile / per;
-  int nn = p.nn;
-  if (p.nn_dev != nullptr) {
-    const int d = __builtin_amdgcn_readfirstlane(*p.nn_dev);
-    nn = d < 0 ? 0 : (d < nn ? d : nn);
-  }
-  if (bi >= nn) return false;
-  const int off = (tile - bi * per) * gc;
-  const int nb = __builtin_amdgcn_readfirstlane(p.nidx[bi]);
-  const bool ok = nb >= 0 && nb < (p.N + 63) / 64;
-  *n0 = ok ? nb * 64 + off : p.npad;
-  *n0y = p.ncompact ? bi * 64 + off : (ok ? *n0 : p.ny);
-  return true;
 }
 
 // |x| of an fp16 value in units of 2^-24 (exact for every finite value; Inf/NaN map above
@@ -538,49 +611,50 @@ __device__ __forceinline__ void self_score_keys(const GemmParams& p, uint64_t* s
 
 // The first na block ids in ascending order, into s_ids[0, na) (na <= BSG_MAX_NBLK / 2): the
 // sequence an ascending sort of the list gives (equal ids are equal, so their order does not
-// show).  The ids go to LDS as unsigned keys 0x7fffffff - id (descending in the id).  A list that
-// is already ascending is copied back; any other is ranked, each id's rank being the number of
-// entries before it in (id asc, list position asc) order, written to
+// show).  Distinct ids of the weight's nblk blocks go through a bitmap; any other list is ranked
+// in LDS as unsigned keys 0x7fffffff - id (descending in the id), each id's rank being the number
+// of entries before it in (id asc, list position asc) order, written to
 // s_ids[BSG_MAX_NBLK / 2 + rank] and copied back.  The rank loop reads the keys as LDS
 // broadcasts and keeps no array, so the kernels' register allocation is not disturbed.  Leaves
-// the copy-back unfenced; the caller's barrier follows.
+// the list unfenced; the caller's barrier follows.
 template <int NT>
-__device__ __forceinline__ void sort_block_list(const int32_t* ids, int na, int* s_ids) {
+__device__ __forceinline__ void sort_block_list(const int32_t* ids, int na, int nblk, int first, int* s_ids) {
   const int tid = threadIdx.x;
+  if (sort_by_bitmap<NT>(ids, na, nblk, first, (uint32_t*)s_ids + BSG_MAX_NBLK / 2,
+                         [&](int r, int id) { s_ids[r] = id; }))
+    return;
   uint32_t* const s_key = (uint32_t*)s_ids;
   for (int i = tid; i < na; i += NT) s_key[i] = (uint32_t)(0x7fffffffLL - (long long)ids[i]);
   __syncthreads();
-  int unsorted = 0;
-  for (int i = tid; i + 1 < na; i += NT) unsorted |= s_key[i] < s_key[i + 1];
-  if (__syncthreads_or(unsorted)) {
-    int* const s_out = s_ids + BSG_MAX_NBLK / 2;
-    for (int i = tid; i < na; i += NT) {
-      const uint32_t ki = s_key[i];
-      int r = 0;
+  int* const s_out = s_ids + BSG_MAX_NBLK / 2;
+  for (int i = tid; i < na; i += NT) {
+    const uint32_t ki = s_key[i];
+    int r = 0;
 #pragma unroll 8
-      for (int j = 0; j < na; ++j) {
-        const uint32_t kj = s_key[j];
-        r += (kj > ki) | ((kj == ki) & (j < i));
-      }
-      s_out[r] = (int)(0x7fffffffLL - (long long)ki);
+    for (int j = 0; j < na; ++j) {
+      const uint32_t kj = s_key[j];
+      r += (kj > ki) | ((kj == ki) & (j < i));
     }
-    __syncthreads();
-    for (int i = tid; i < na; i += NT) s_ids[i] = s_out[i];
-  } else {
-    // each thread rewrites only the entries it read
-    for (int i = tid; i < na; i += NT) s_ids[i] = (int)(0x7fffffffLL - (long long)s_key[i]);
+    s_out[r] = (int)(0x7fffffffLL - (long long)ki);
   }
+  __syncthreads();
+  for (int i = tid; i < na; i += NT) s_ids[i] = s_out[i];
+}
+
+// This thread's entry of a list the kernel is to sort, requested at kernel entry (a list whose
+// length is on the device is read once the length is known).
+__device__ __forceinline__ int list_entry_of_thread(const GemmParams& p) {
+  return p.sort_list && p.na_dev == nullptr && (int)threadIdx.x < p.na ? p.idx[threadIdx.x] : 0;
 }
 
 // Stage this call's active-block list in LDS (list copy, bitmap compaction, top-k of block
 // scores or identity) and return its length.  Ends with a barrier.  s_ids is 16-byte aligned
 // and holds BSG_MAX_NBLK ids; the top-k stages its keys in the first half and its ranks in the
-// second (up to 512 blocks).  ONE_D: the in-kernel sort of a 1-D list (p.sort_list) is compiled
-// in (the 2-D forms have none).  SEL: the in-GEMM top-k (MODE_TOPK) is, and SELF_SCORE its
+// second (up to 512 blocks).  SEL: the in-GEMM top-k (MODE_TOPK) is, and SELF_SCORE its
 // self-scored form (MODE_TOPK_SELF): the selection instantiations only (KernelEntry::f16_sel),
 // which alone are launched in those modes.
-template <int NT, bool ONE_D, bool SEL = false, bool SELF_SCORE = false>
-__device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids, int* s_scan) {
+template <int NT, bool SEL = false, bool SELF_SCORE = false>
+__device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids, int* s_scan, int first) {
   const int tid = threadIdx.x;
   int na = 0;
   bool ranked = false;
@@ -603,9 +677,10 @@ __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids,
     if (p.na_dev != nullptr) {
       const int d = *p.na_dev;
       na = d < 0 ? 0 : (d < na ? d : na);
+      if (p.sort_list && tid < na) first = p.idx[tid];
     }
-    if (ONE_D && p.sort_list)
-      sort_block_list<NT>(p.idx, __builtin_amdgcn_readfirstlane(na), s_ids);
+    if (p.sort_list)
+      sort_block_list<NT>(p.idx, __builtin_amdgcn_readfirstlane(na), p.nblk, first, s_ids);
     else
       for (int i = tid; i < na; i += NT) s_ids[i] = p.idx[i];
   } else if (p.mode == MODE_BITMAP) {
@@ -755,13 +830,14 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   int tile, sk;
   tile_of_group(p.split_k, &tile, &sk);
   const int S = p.split_k;
+  const int first = list_entry_of_thread(p);
   int n0, n0y;
-  if (!tile_columns<N2D>(p, tile, 16 * NSUB, &n0, &n0y)) return;
+  if (!tile_columns<N2D, NT>(p, tile, 16 * NSUB, &n0, &n0y)) return;
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, !N2D, SEL, SEL && BTT == 1>(p, s_ids, s_misc);
+  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
   BSG_TL(1);
 
   // This wave's contiguous slice [pbeg, pend) of the list.
@@ -925,13 +1001,14 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
   int tile, sk;
   tile_of_group(p.split_k, &tile, &sk);
   const int S = p.split_k;
+  const int first = list_entry_of_thread(p);
   int n0, n0y;
-  if (!tile_columns<N2D>(p, tile, 16 * CS, &n0, &n0y)) return;
+  if (!tile_columns<N2D, NT>(p, tile, 16 * CS, &n0, &n0y)) return;
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, !N2D, SEL, SEL && BTT == 1>(p, s_ids, s_misc);
+  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
   BSG_TL(1);
 
   // The work-group's contiguous slice of the list (all its waves walk it together).
@@ -1090,13 +1167,14 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_fma_kernel(GemmParams p) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = blockIdx.x;
+  const int first = list_entry_of_thread(p);
   int n0, n0y;
-  if (!tile_columns<N2D>(p, tile, 16 * NSUB, &n0, &n0y)) return;
+  if (!tile_columns<N2D, NT>(p, tile, 16 * NSUB, &n0, &n0y)) return;
   const int y0 = blockIdx.y * BT;
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, !N2D>(p, s_ids, s_misc);
+  const int na = stage_block_list<NT>(p, s_ids, s_misc, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * w) / WPG);
   const int pend = (int)(((int64_t)na * (w + 1)) / WPG);
@@ -1301,11 +1379,12 @@ __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p)
   tile_of_group(1, &tile, &sk);
   int st, nv;
   vt_columns(tile, p.n_tiles, p.npad >> 4, &st, &nv);
+  const int first = list_entry_of_thread(p);
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, true, SEL, SEL && BTT == 1>(p, s_ids, s_misc);
+  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * b) / WB);
   const int pend = (int)(((int64_t)na * (b + 1)) / WB);
@@ -1437,11 +1516,12 @@ __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   tile_of_group(1, &tile, &sk);
   int st, nv;
   vt_columns(tile, p.n_tiles, p.npad >> 4, &st, &nv);
+  const int first = list_entry_of_thread(p);
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, true, SEL, SEL && BTT == 1>(p, s_ids, s_misc);
+  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * w) / WB);
   const int pend = (int)(((int64_t)na * (w + 1)) / WB);

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, true>(p, s_ids, s_misc);
+  const int na = stage_block_list<NT>(p, s_ids, s_misc, list_entry_of_thread(p));
   BSG_TL(1);
 
   const int blk_bytes = p.npad * 128;

@@ -751,6 +751,9 @@ struct LaunchExtras {
   int32_t nn = 0;
   const int32_t* nn_dev = nullptr;
   int ncompact = 0;
+  // the output-block list has nn_list entries in any order; the kernel sorts it into nidx_out
+  int32_t nn_list = 0;
+  int32_t* nidx_out = nullptr;
   // Fixed split-K storage (the allocation-free entry point): counters and partials at these
   // addresses, with room for cnt_cap_tiles counters and part_cap_bytes of partials, instead of
   // being carved from ws.
@@ -865,11 +868,15 @@ int launch_gemm(int mode, const void* x, int64_t ldx, int64_t bt, int64_t K, con
   p.idx_out = ex.idx_out;
   p.na_out = ex.na_out;
   p.keyed = ex.score_keyed && bt <= 64;
-  p.sort_list = mode == MODE_LIST && ex.sort_list && ex.nidx == nullptr;
+  p.sort_list = mode == MODE_LIST && ex.sort_list;
   p.nidx = ex.nidx;
   p.nn_dev = ex.nn_dev;
   p.nn = ex.nn;
   p.ncompact = ex.ncompact;
+  if (ex.nidx_out != nullptr) {  // the 2-D forms' use of these fields (GemmParams)
+    p.idx_out = ex.nidx_out;
+    p.keyed = ex.nn_list;
+  }
   p.tl = timeline_slot((int64_t)n_tiles * pl.split_k * ygroups);
 
   dim3 grid((unsigned)(n_tiles * pl.split_k), (unsigned)ygroups, 1);
@@ -1028,25 +1035,52 @@ int bsg_gemm_dense(const void* x, int64_t ldx, int64_t bt, int64_t K, const void
                      ws_bytes, plan, stream);
 }
 
-int bsg_gemm_2d(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
-                const int32_t* active_blocks, int32_t num_active, const int32_t* num_active_dev,
-                const int32_t* n_blocks, int32_t num_n, const int32_t* num_n_dev, int compact, void* y,
-                int64_t ldy, int dtype, void* ws, int64_t ws_bytes, const bsg_plan* plan, void* stream) {
+static int gemm_2d_run(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
+                       const int32_t* active_blocks, int32_t num_active, const int32_t* num_active_dev,
+                       int32_t num_n, void* y, int64_t ldy, int dtype, void* ws, int64_t ws_bytes,
+                       const bsg_plan* plan, void* stream, const LaunchExtras& ex) {
   if (num_n < 0 || num_n > cdiv(N, 64))
     return fail(BSG_ERR_ARG, "2-D: num_n=%d outside [0, ceil(N/64)] (N=%lld)", num_n, (long long)N);
   if (num_n == 0)  // no output block: only the checks run, nothing is written
-    return check_common(x, ldx, bt, K, wp, N, y, ldy, dtype, compact ? 0 : N);
-  if (!n_blocks) return fail(BSG_ERR_ARG, "2-D: n_blocks is null");
-  LaunchExtras ex;
-  ex.nidx = n_blocks;
-  ex.nn = num_n;
-  ex.nn_dev = num_n_dev;
-  ex.ncompact = compact != 0;
+    return check_common(x, ldx, bt, K, wp, N, y, ldy, dtype, ex.ncompact ? 0 : N);
+  if (!ex.nidx) return fail(BSG_ERR_ARG, "2-D: n_blocks is null");
   if (active_blocks == nullptr && num_active_dev == nullptr)
     return launch_gemm(MODE_DENSE, x, ldx, bt, K, wp, N, nullptr, 0, nullptr, nullptr, 0, y, ldy, dtype, ws,
                        ws_bytes, plan, stream, ex);
   return launch_gemm(MODE_LIST, x, ldx, bt, K, wp, N, active_blocks, num_active, num_active_dev, nullptr, 0, y,
                      ldy, dtype, ws, ws_bytes, plan, stream, ex);
+}
+
+int bsg_gemm_2d(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
+                const int32_t* active_blocks, int32_t num_active, const int32_t* num_active_dev,
+                const int32_t* n_blocks, int32_t num_n, const int32_t* num_n_dev, int compact, void* y,
+                int64_t ldy, int dtype, void* ws, int64_t ws_bytes, const bsg_plan* plan, void* stream) {
+  LaunchExtras ex;
+  ex.nidx = n_blocks;
+  ex.nn = num_n;
+  ex.nn_dev = num_n_dev;
+  ex.ncompact = compact != 0;
+  return gemm_2d_run(x, ldx, bt, K, wp, N, active_blocks, num_active, num_active_dev, num_n, y, ldy, dtype, ws,
+                     ws_bytes, plan, stream, ex);
+}
+
+int bsg_gemm_2d_sorted(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
+                       const int32_t* active_blocks, int32_t num_active, int sort_active, const int32_t* n_blocks,
+                       int32_t num_n_list, int32_t num_n, int32_t* n_sorted_out, int compact, void* y, int64_t ldy,
+                       int dtype, void* ws, int64_t ws_bytes, const bsg_plan* plan, void* stream) {
+  if (n_sorted_out != nullptr && (num_n_list < num_n || num_n_list > BSG_2D_SORT_MAX))
+    return fail(num_n_list < num_n ? BSG_ERR_ARG : BSG_ERR_UNSUPPORTED,
+                "2-D in-kernel sort: a list of %d output blocks, %d taken (at most %d)", num_n_list, num_n,
+                BSG_2D_SORT_MAX);
+  LaunchExtras ex;
+  ex.nidx = n_blocks;
+  ex.nn = num_n;
+  ex.ncompact = compact != 0;
+  ex.sort_list = sort_active != 0;
+  ex.nn_list = num_n_list;
+  ex.nidx_out = n_sorted_out;
+  return gemm_2d_run(x, ldx, bt, K, wp, N, active_blocks, num_active, nullptr, num_n, y, ldy, dtype, ws, ws_bytes,
+                     plan, stream, ex);
 }
 
 int bsg_scatter_nblocks(const void* compact, int64_t ldc, int64_t bt, const int32_t* n_blocks, int32_t num_n,
