@@ -292,8 +292,8 @@ int bsg_select_gemm(const void* x, int64_t ldx, int64_t bt, int64_t K, int32_t k
  * energy budget.  idx_out, *na_out and ratio_out receive exactly what bsg_select_topk gives for
  * the same x and opts (idx_out needs room for floor(K/64) ids under an energy budget, min(k,
  * floor(K/64)) otherwise).  Two launches (fp64 order keys of the block scores, then the GEMM,
- * whose work-groups rank the keys themselves) when there is no energy budget, no ratio_out, the
- * dtype is fp16 and the plan's waves can rank the blocks (as bsg_select_gemm); otherwise three
+ * whose work-groups rank the keys themselves and scan the energies of a budget or ratio) when the
+ * plan's waves can rank the blocks (as bsg_select_gemm); otherwise three
  * (scores, one-work-group rank, GEMM on the device count).  opts->score == BSG_SCORE_L1 is
  * bsg_select_gemm.  Workspace as bsg_select_gemm: bsg_select_workspace_bytes(K) bytes for the
  * selector, then the GEMM's. */

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import bsa_mi355x as bsa
-from bsa_mi355x.select import select_gemm_packed
+from bsa_mi355x.select import select_gemm_packed, select_gemm_rule_packed
 from helpers import assert_close, case, to_dev
 from oracle import bsg_oracle as orc
 
@@ -535,3 +535,51 @@ def test_rule_select_gemm_ranks_a_nan_block_first(dev):
         want, _, _ = orc.select_scored_ref(x, 3, score)
         assert c == 3 and np.array_equal(got, [10, 20, 40]) and np.array_equal(want, [10, 20, 40])
         assert np.array_equal(s_idx, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bt,kdim,plan", [
+    (5, 64, (1, 16, 2, 4, 16, 1)),        # one block
+    (3, 4096, (1, 16, 1, 4, 16, 1)),      # one wave
+    (16, 4160, (2, 16, 2, 8, 16, 1)),     # 65 blocks, split-K
+    (9, 4136, (1, 48, 4, 4, 16, 5)),      # a partial last block
+    (30, 8192, (1, 32, 4, 4, 32, 7)),     # 128 blocks
+    (64, 8256, (1, 48, 8, 2, 64, 7)),     # 129 blocks
+    (40, 11008, (2, 16, 8, 4, 64, 4)),    # 172 blocks
+    (20, 13824, (1, 16, 8, 4, 32, 6)),    # 216 blocks
+])
+def test_energy_budget_inside_the_gemm(dev, dtype, bt, kdim, plan):
+    """The budget's kept ids, count and ratio are those of the separate selector, bit for bit, and
+    the GEMM is the one on that list: k from 0 past the block count, budgets from none to all, equal
+    energies (sums that meet the budget exactly), zero, infinite and NaN energies."""
+    nb, n = kdim // 64, 176
+    rng = np.random.default_rng(kdim + bt)
+    base = rng.laplace(0, 0.05, size=(bt, kdim)) * np.exp(0.7 * rng.normal(size=kdim))
+    cases = {"plain": base, "equal": np.full((bt, kdim), 0.25), "zero": np.zeros((bt, kdim))}
+    for name, v in (("inf", np.inf), ("nan", np.nan)):
+        bad = base.copy()
+        bad[bt // 2, 64 * (nb // 2)] = v
+        cases[name] = bad
+    w = torch.from_numpy(rng.normal(0, 0.02, size=(n, kdim)).astype(np.float32)).to(dtype).to(dev)
+    packed = bsa.pack_weight(w)
+    p = bsa.Plan(*plan)
+    for name, x in cases.items():
+        xt = torch.from_numpy(x.astype(np.float32)).to(dtype).to(dev)
+        for k, keep in ((0, 0.5), (1, 0.5), (nb // 2 + 1, 0.5), (nb + 3, 0.5), (1, 0.0), (1, 0.001), (1, 1.0), (2, 0.97)):
+            print(f"budget {dtype} bt={bt} K={kdim} plan={plan} {name} k={k} keep={keep}", flush=True)
+            ids = torch.full((nb,), -1, dtype=torch.int32, device=dev)
+            y = torch.empty(bt, n, dtype=dtype, device=dev)
+            ratio = torch.full((1,), -1.0, device=dev)
+            _, cnt, _ = select_gemm_rule_packed(xt, packed, n, k, y, score="energy", energy_keep=keep, plan=p,
+                                                idx_out=ids, ratio_out=ratio)
+            s_ids, s_cnt, s_ratio = bsa.select_topk(xt, k, score="energy", energy_keep=keep,
+                                                    ratio_out=torch.full((1,), -2.0, device=dev))
+            c = int(cnt.item())
+            assert c == int(s_cnt.item()) and torch.equal(ids[:c], s_ids[:c]) and bool((ids[c:] == -1).all())
+            assert torch.equal(ratio.view(torch.int32), s_ratio.view(torch.int32))
+            if name in ("plain", "equal"):
+                want, keep_n, wr = orc.select_scored_ref(xt.float().cpu().numpy(), k, "energy", energy_keep=keep)
+                assert c == keep_n and np.array_equal(ids[:c].cpu().numpy(), want)
+            ref = torch.empty_like(y)
+            bsa.gemm_packed(xt, packed, n, s_ids[:c].contiguous(), ref, plan=p, num_active=c)
+            assert torch.equal(y.view(torch.int16), ref.view(torch.int16))

@@ -301,8 +301,8 @@ def select_gemm_rule_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int,
                             ) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Selection by the reference's rules (select_topk's options, RRD:90-176) + the GEMM on the
     kept blocks, one library call (bsg_select_gemm_rule): the kept ids, count and ratio are those
-    select_topk gives for the same x and options, all on the device.  Two launches when the GEMM
-    ranks the fp64 score keys itself (no energy budget, no ratio, fp16), else three.  Returns
+    select_topk gives for the same x and options, all on the device.  Two launches when the plan's
+    waves can rank the fp64 score keys, else three.  Returns
     (idx int32 with room for the capacity, count [1], ratio [1] or None)."""
     c = prepare_select_gemm_rule(x2d, packed, n_dim, k, y2d, score, block_prior, prior_alpha, prior_eps,
                                  channel_scale, energy_keep, plan, idx_out, count_out, ratio_out, workspace_prefix)

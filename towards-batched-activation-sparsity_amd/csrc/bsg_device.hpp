@@ -21,12 +21,20 @@ struct GemmParams {
   void* y;
   const int32_t* idx;
   const int32_t* na_dev;
-  const uint8_t* bitmap;
+  union {
+    const uint8_t* bitmap;  // MODE_BITMAP
+    float* ratio_out;       // MODE_TOPK_BUDGET: the kept energy fraction (null: not published)
+  };
   float* part;
   uint32_t* cnt;
   int64_t ldx;
   int64_t ldy;
-  int32_t bt, K, N, npad, nblk, nbm, na, mode, split_k, n_tiles, x_bytes, y_fast;
+  int32_t bt, K, N, npad, nblk;
+  union {
+    int32_t nbm;        // MODE_BITMAP: entries of the bitmap
+    float energy_keep;  // MODE_TOPK_BUDGET: the energy fraction to keep (0: none)
+  };
+  int32_t na, mode, split_k, n_tiles, x_bytes, y_fast;
   // MODE_TOPK: exact-L1 block scores (na = k), whether they fit the unique-key order, and where
   // work-group (0, 0) publishes the kept list and its count (null: not published)
   const uint64_t* scores;
@@ -54,12 +62,14 @@ typedef void (*GemmFn)(GemmParams);
 enum { KIND_KSPLIT = 1, KIND_XLDS = 2, KIND_FMA = 3, KIND_XLDS_KH = 4, KIND_VT = 5, KIND_VT1 = 6, KIND_VT1X = 7, KIND_ROWS = 8 };
 
 // 1-D and, for tiles of at most 64 columns per work-group, 2-D (active output blocks) entries.
-// f16_sel: the fp16 1-D form compiled with the in-GEMM top-k (MODE_TOPK; on 16-row tiles also
-// the self-scored MODE_TOPK_SELF), for the MFMA kinds (null for kind 3).  The other forms leave
-// that code out: carried in every kernel it cost every plain launch 0.1-0.2 us.
+// f16_sel, bf16_sel: the 1-D form compiled with the in-GEMM top-k (MODE_TOPK; in fp16 on 16-row
+// tiles also the self-scored MODE_TOPK_SELF), for the MFMA kinds (null for kinds 3 and 8); f16_bud,
+// bf16_bud: with the top-k under an energy budget (MODE_TOPK_BUDGET).  Every form leaves out what it
+// does not run: the top-k carried in every kernel cost every plain launch 0.1-0.2 us, and the
+// budget carried in the top-k kernels drained the loops of some (decode step 579 -> 658 us).
 struct KernelEntry {
   int kind, rows, nsub, wpg, depth;
-  GemmFn f16, bf16, f16_2d, bf16_2d, f16_sel;
+  GemmFn f16, bf16, f16_2d, bf16_2d, f16_sel, bf16_sel, f16_bud, bf16_bud;
 };
 
 // A translation unit's slice of the instantiated tile set.
@@ -131,10 +141,13 @@ constexpr int kRsrcWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, 
 
 // MODE_TOPK: the GEMM ranks block scores an earlier launch wrote.  MODE_TOPK_SELF: every
 // work-group also computes those scores itself from x (fp16, at most BSG_SELF_MAX_ROWS rows).
-enum { MODE_LIST = 0, MODE_BITMAP = 1, MODE_DENSE = 2, MODE_TOPK = 3, MODE_TOPK_SELF = 4 };
+// MODE_TOPK_BUDGET: as MODE_TOPK, the kept count grown to an energy budget (energy_budget).
+enum { MODE_LIST = 0, MODE_BITMAP = 1, MODE_DENSE = 2, MODE_TOPK = 3, MODE_TOPK_SELF = 4, MODE_TOPK_BUDGET = 5 };
 // A GEMM ranks block scores itself (MODE_TOPK) up to this many blocks: keys and ranks fit its
 // block-list buffer, and a one-wave work-group flags at most 8 per thread.
 #define BSG_TOPK_MAX_NBLK 512
+// What selection code a kernel form carries (KernelEntry).
+enum { SEL_NONE = 0, SEL_TOPK = 1, SEL_BUDGET = 2 };
 #define BSG_SELF_MAX_ROWS 8
 
 // The 2-D kernels sort an output-block list of up to this many entries themselves.
@@ -292,6 +305,78 @@ __device__ __forceinline__ void pad_scores(S* s_sc, int nb) {
   if (tid < ((nb + 15) & ~15) - nb) s_sc[nb + tid] = S(0);
 }
 
+// One DPP row shift (row_shr:n = 0x110 + n) of a 64-bit value: lane i of each 16-lane row
+// reads lane i - n of the same row, and 0 where that lane lies outside the row.
+template <int CTRL>
+__device__ __forceinline__ uint64_t u64_row_shr(uint64_t x) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, 0xf, 0xf, true);
+  return ((uint64_t)hi << 32) | lo;
+}
+
+// x plus lane i - n's x within the same 16-lane row (0 outside it), in fp64.
+template <int CTRL>
+__device__ __forceinline__ double f64_row_shr(double x) {
+  return x + __builtin_bit_cast(double, u64_row_shr<CTRL>(__builtin_bit_cast(uint64_t, x)));
+}
+
+// Lane `src`'s fp64 value (src wave-uniform).
+__device__ __forceinline__ double f64_readlane(double x, int src) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  return __builtin_bit_cast(
+      double, ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), src) << 32) |
+                  (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, src));
+}
+
+// Blocks an energy budget keeps, by one wave: s_e[0, nb) holds the blocks' energies in rank order
+// and is overwritten with their running sums; the count is k0 when those ranks already hold `keep` of
+// the total, else up to the first rank whose running sum reaches it (at most cap); *ratio (by
+// lane 0, when not null) receives the kept fraction.  Every caller sums in the same order (64
+// ranks at a time, DPP scans within 16-lane rows, then the rows before), so the rank launch and a
+// GEMM that ranks for itself keep the same blocks.
+__device__ __forceinline__ int energy_budget(double* s_e, int nb, int k0, int cap, float keep, float* ratio) {
+  const int lane = threadIdx.x & 63;
+  double before = 0.0;
+  for (int r0 = 0; r0 < nb; r0 += 64) {
+    double c = r0 + lane < nb ? s_e[r0 + lane] : 0.0;
+    c = f64_row_shr<0x111>(c);
+    c = f64_row_shr<0x112>(c);
+    c = f64_row_shr<0x114>(c);
+    c = f64_row_shr<0x118>(c);
+    const double r1 = f64_readlane(c, 15), r2 = r1 + f64_readlane(c, 31), r3 = r2 + f64_readlane(c, 47);
+    c += lane < 16 ? 0.0 : lane < 32 ? r1 : lane < 48 ? r2 : r3;
+    c += before;
+    before = f64_readlane(c, 63);
+    if (r0 + lane < nb) s_e[r0 + lane] = c;
+  }
+  const double total = before > 1e-12 ? before : 1e-12;
+  int kept = k0;
+  if (keep > 0.f && k0 > 0 && s_e[k0 - 1] / total < (double)keep) {
+    const double thr = (double)keep * total;
+    int first = nb;
+    for (int r0 = 0; r0 < nb; r0 += 64) {
+      const uint64_t m = __ballot(r0 + lane < nb && s_e[r0 + lane] >= thr);
+      if (m != 0) {
+        first = r0 + __builtin_ctzll(m);
+        break;
+      }
+    }
+    kept = first + 1;
+    kept = kept < k0 ? k0 : (kept > cap ? cap : kept);
+  }
+  if (ratio != nullptr && lane == 0) *ratio = kept > 0 ? (float)(s_e[kept - 1] / total) : 0.f;
+  return kept;
+}
+
+// An energy budget for topk_l1_list: the blocks' energies, the fraction to keep, the most blocks it
+// may keep and where the kept fraction goes (null: nowhere).
+struct EnergyBudget {
+  const double* energy;
+  float keep;
+  int cap;
+  float* ratio;
+};
+
 // Top-k of nb exact-L1 block scores (global memory, written by an earlier kernel on the
 // stream): ranked (score desc, id asc), the first k kept, their ids handed to emit(position,
 // id) in ascending id order.  keyed: every score is below 2^53, so (score << 11) | (2047 - id)
@@ -300,12 +385,17 @@ __device__ __forceinline__ void pad_scores(S* s_sc, int nb) {
 // scores ahead of its block and adds the count to the block's rank in LDS.  s_key holds nb
 // keys rounded up to 16, s_rank nb ints; per-wave ballots of the kept flags then give ascending
 // positions.  Returns min(k, nb).  No thread reads s_key after the ranking barrier, so emit may
-// overwrite s_key (not s_rank, which waves still read while others emit).
-template <int NT, typename Emit>
+// overwrite s_key (not s_rank, which waves still read while others emit).  BUDGET: the count grows
+// from min(k, nb) to the budget's; the energies then pass through s_key's storage in rank order,
+// and s_rank holds one more int.
+template <int NT, bool BUDGET = false, typename Emit>
 __device__ __forceinline__ int topk_l1_list(const uint64_t* scores, int nb, int k, bool keyed, uint64_t* s_key,
-                                            int* s_rank, Emit emit, bool staged = false) {
+                                            int* s_rank, Emit emit, bool staged = false,
+                                            EnergyBudget budget = {}) {
   constexpr int W = NT / 64;
   const int tid = threadIdx.x, lane = tid & 63;
+  double e0 = 0.0;  // this thread's first energy, requested with the scores
+  if constexpr (BUDGET) e0 = tid < nb ? budget.energy[tid] : 0.0;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nb16 = (nb + 15) & ~15;
   // staged: s_key already holds the keys and pads (self_score_keys)
@@ -345,7 +435,19 @@ __device__ __forceinline__ int topk_l1_list(const uint64_t* scores, int nb, int 
   // kept flags of each 64-block group in turn and keeps the running count, so the position of
   // block j is the kept count before its group plus the kept lanes below it; wave g % W emits
   // group g.  No barrier, and the only LDS reads are of s_rank.
-  const int kk = k < nb ? k : nb;
+  int kk = k < nb ? k : nb;
+  if constexpr (BUDGET) {
+    double* const s_e = (double*)s_key;
+    for (int j = tid; j < nb; j += NT) s_e[s_rank[j]] = j == tid ? e0 : budget.energy[j];
+    __syncthreads();
+    if (w == 0) {
+      const int kept =
+          energy_budget(s_e, nb, kk < budget.cap ? kk : budget.cap, budget.cap, budget.keep, budget.ratio);
+      if (lane == 0) s_rank[nb] = kept;
+    }
+    __syncthreads();
+    kk = s_rank[nb];
+  }
   int before = 0;
 #pragma unroll 1
   for (int g = 0; 64 * g < nb; ++g) {
@@ -531,15 +633,6 @@ __device__ __forceinline__ double f16x8_abs_sum(u32x4 v) {
   return ((h(v.x, 0) + h(v.x, 1)) + (h(v.y, 0) + h(v.y, 1))) + ((h(v.z, 0) + h(v.z, 1)) + (h(v.w, 0) + h(v.w, 1)));
 }
 
-// One DPP row shift (row_shr:n = 0x110 + n) of a 64-bit value: lane i of each 16-lane row
-// reads lane i - n of the same row, and 0 where that lane lies outside the row.
-template <int CTRL>
-__device__ __forceinline__ uint64_t u64_row_shr(uint64_t x) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, 0xf, 0xf, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, 0xf, 0xf, true);
-  return ((uint64_t)hi << 32) | lo;
-}
-
 // The 64-bit value of lane `src` of the wave.
 __device__ __forceinline__ uint64_t u64_lane(uint64_t x, int src) {
   const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)x, src, 64);
@@ -650,28 +743,28 @@ __device__ __forceinline__ int list_entry_of_thread(const GemmParams& p) {
 // Stage this call's active-block list in LDS (list copy, bitmap compaction, top-k of block
 // scores or identity) and return its length.  Ends with a barrier.  s_ids is 16-byte aligned
 // and holds BSG_MAX_NBLK ids; the top-k stages its keys in the first half and its ranks in the
-// second (up to 512 blocks).  SEL: the in-GEMM top-k (MODE_TOPK) is, and SELF_SCORE its
-// self-scored form (MODE_TOPK_SELF): the selection instantiations only (KernelEntry::f16_sel),
-// which alone are launched in those modes.
-template <int NT, bool SEL = false, bool SELF_SCORE = false>
+// second (up to 512 blocks).  SEL: only the in-GEMM top-k is compiled in (SELF_SCORE: also its
+// self-scored form), in the selection forms of KernelEntry, which are launched in those modes only;
+// without the list, bitmap and dense branches beside it the selection + GEMM calls take 2-4% less.
+template <int NT, int SEL = SEL_NONE, bool SELF_SCORE = false>
 __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids, int* s_scan, int first) {
   const int tid = threadIdx.x;
   int na = 0;
-  bool ranked = false;
-  if constexpr (SEL) {
-    if (p.mode == MODE_TOPK || (SELF_SCORE && p.mode == MODE_TOPK_SELF)) {
-      // Every work-group ranks the scores itself (identically), so the list needs no other
-      // launch; keys and ranks are staged in the list buffer and overwritten by the kept ids.
-      // MODE_TOPK_SELF computes the scores here too, so the selection needs no launch of its own.
-      const bool self = SELF_SCORE && p.mode == MODE_TOPK_SELF;
-      if (self) self_score_keys<NT>(p, (uint64_t*)s_ids);
-      na = topk_l1_list<NT>(p.scores, p.nblk, p.na, p.keyed != 0, (uint64_t*)s_ids, s_ids + BSG_MAX_NBLK / 2,
-                            [&](int pos, int id) { s_ids[pos] = id; }, self);
-      ranked = true;
-    }
-  }
-  if (ranked) {
-    // the kept list is staged
+  if constexpr (SEL == SEL_TOPK) {
+    // Launched in MODE_TOPK and MODE_TOPK_SELF only.  Every work-group ranks the scores itself
+    // (identically), so the list needs no other launch; keys and ranks are staged in the list
+    // buffer and overwritten by the kept ids.  MODE_TOPK_SELF computes the scores here too, so the
+    // selection needs no launch of its own.
+    const bool self = SELF_SCORE && p.mode == MODE_TOPK_SELF;
+    if (self) self_score_keys<NT>(p, (uint64_t*)s_ids);
+    na = topk_l1_list<NT>(p.scores, p.nblk, p.na, p.keyed != 0, (uint64_t*)s_ids, s_ids + BSG_MAX_NBLK / 2,
+                          [&](int pos, int id) { s_ids[pos] = id; }, self);
+  } else if constexpr (SEL == SEL_BUDGET) {
+    // launched in MODE_TOPK_BUDGET only; the energies follow the scores, work-group (0, 0) publishes
+    na = topk_l1_list<NT, true>(p.scores, p.nblk, p.na, false, (uint64_t*)s_ids, s_ids + BSG_MAX_NBLK / 2,
+                                [&](int pos, int id) { s_ids[pos] = id; }, false,
+                                {(const double*)(p.scores + p.nblk), p.energy_keep, p.K / BSG_BLOCK_K,
+                                 blockIdx.x == 0 && blockIdx.y == 0 ? p.ratio_out : nullptr});
   } else if (p.mode == MODE_LIST) {
     na = p.na;
     if (p.na_dev != nullptr) {
@@ -700,7 +793,7 @@ __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids,
   }
   na = __builtin_amdgcn_readfirstlane(na);
   __syncthreads();
-  if (SEL && ranked && p.idx_out != nullptr && blockIdx.x == 0 && blockIdx.y == 0) {
+  if (SEL != SEL_NONE && p.idx_out != nullptr && blockIdx.x == 0 && blockIdx.y == 0) {
     for (int i = tid; i < na; i += NT) p.idx_out[i] = s_ids[i];
     if (tid == 0) *p.na_out = na;
   }
@@ -813,7 +906,7 @@ __device__ __forceinline__ void splitk_finish(const GemmParams& p, size_t tile_l
 // the work-group's share of the block list into contiguous slices and are reduced through LDS
 // in wave order.  Each wave loads its own X fragments.  Best when bt is small (the X fragments
 // are few) and many narrow column tiles are needed to fill the chip.
-template <typename T, int BTT, int NSUB, int WPG, int DEPTH, bool N2D, bool SEL = false>
+template <typename T, int BTT, int NSUB, int WPG, int DEPTH, bool N2D, int SEL = SEL_NONE>
 __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   constexpr int NT = 64 * WPG;
   constexpr int F = BTT * NSUB;
@@ -837,7 +930,7 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
   BSG_TL(1);
 
   // This wave's contiguous slice [pbeg, pend) of the list.
@@ -980,7 +1073,7 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
 // (WK = 2): 2*WC waves, column group x 32-channel half of every block, so each wave issues half
 // the MFMAs and LDS reads of a block and two waves share each SIMD, overlapping one wave's
 // barrier and LDS waits with the other's MFMAs; the halves are summed through LDS at the end.
-template <typename T, int BTT, int NSUB, int WC, int WK, int DEPTH, bool N2D, bool SEL = false>
+template <typename T, int BTT, int NSUB, int WC, int WK, int DEPTH, bool N2D, int SEL = SEL_NONE>
 __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p) {
   constexpr int WPG = WC * WK;
   constexpr int NT = 64 * WPG;
@@ -1008,7 +1101,7 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
   BSG_TL(1);
 
   // The work-group's contiguous slice of the list (all its waves walk it together).
@@ -1361,7 +1454,7 @@ __device__ __forceinline__ void vt_columns(int t, int G, int T, int* first, int*
 // KH = 1 (kind 6): no channel-half split; each of the WB waves loads both halves of every
 // weight subtile and activation row tile of its blocks (the two halves of an activation row are
 // one 128-byte line, requested back to back by one wave).
-template <typename T, int BTT, int NSUB, int WB, int DEPTH, int KH = 2, bool SEL = false>
+template <typename T, int BTT, int NSUB, int WB, int DEPTH, int KH = 2, int SEL = SEL_NONE>
 __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p) {
   constexpr int NW = KH * WB;
   constexpr int NT = 64 * NW;
@@ -1384,7 +1477,7 @@ __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p)
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * b) / WB);
   const int pend = (int)(((int64_t)na * (b + 1)) / WB);
@@ -1500,7 +1593,7 @@ __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p)
 // for four block-slice waves at 64 rows; the wave reduction reuses each wave's own slots.  A
 // separate kernel from kind 6 so that kind 6's generated code stays as it is (its schedules
 // change with unrelated code in the same function).
-template <typename T, int BTT, int NSUB, int WB, int DEPTH, bool SEL = false>
+template <typename T, int BTT, int NSUB, int WB, int DEPTH, int SEL = SEL_NONE>
 __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   constexpr int NT = 64 * WB;
   constexpr int F = BTT * NSUB;
@@ -1521,7 +1614,7 @@ __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL && BTT == 1>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * w) / WB);
   const int pend = (int)(((int64_t)na * (w + 1)) / WB);
@@ -1675,47 +1768,50 @@ constexpr GemmFn kernel_2d() {
   }
 }
 
-// The selection form (fp16, 1-D, in-GEMM top-k) of a tile of the MFMA kinds.
-template <int KIND, int B, int S, int W, int D>
+// A selection form (1-D, in-GEMM top-k, SEL_TOPK or SEL_BUDGET) of a tile of the MFMA kinds.
+template <int KIND, typename T, int SEL, int B, int S, int W, int D>
 constexpr GemmFn kernel_sel() {
   if constexpr (KIND == KIND_KSPLIT) {
-    return bsg_gemm_kernel<_Float16, B, S, W, D, false, true>;
+    return bsg_gemm_kernel<T, B, S, W, D, false, SEL>;
   } else if constexpr (KIND == KIND_XLDS) {
-    return bsg_gemm_xl_kernel<_Float16, B, S, W, 1, D, false, true>;
+    return bsg_gemm_xl_kernel<T, B, S, W, 1, D, false, SEL>;
   } else if constexpr (KIND == KIND_XLDS_KH) {
-    return bsg_gemm_xl_kernel<_Float16, B, S, W / 2, 2, D, false, true>;
+    return bsg_gemm_xl_kernel<T, B, S, W / 2, 2, D, false, SEL>;
   } else if constexpr (KIND == KIND_VT) {
-    return bsg_gemm_vt_kernel<_Float16, B, S, W / 2, D, 2, true>;
+    return bsg_gemm_vt_kernel<T, B, S, W / 2, D, 2, SEL>;
   } else if constexpr (KIND == KIND_VT1) {
-    return bsg_gemm_vt_kernel<_Float16, B, S, W, D, 1, true>;
+    return bsg_gemm_vt_kernel<T, B, S, W, D, 1, SEL>;
   } else {
-    return bsg_gemm_vtx_kernel<_Float16, B, S, W, D, true>;
+    return bsg_gemm_vtx_kernel<T, B, S, W, D, SEL>;
   }
 }
 
+#define BSG_SEL_FORMS(KIND, B, S, W, D)                                                          \
+  kernel_sel<KIND, _Float16, SEL_TOPK, B, S, W, D>(), kernel_sel<KIND, __bf16, SEL_TOPK, B, S, W, D>(), \
+      kernel_sel<KIND, _Float16, SEL_BUDGET, B, S, W, D>(), kernel_sel<KIND, __bf16, SEL_BUDGET, B, S, W, D>()
 #define BSG_K(B, S, W, D)                                                                                          \
   {KIND_KSPLIT, 16 * B, S, W, D, bsg_gemm_kernel<_Float16, B, S, W, D, false>, bsg_gemm_kernel<__bf16, B, S, W, D, false>, \
    kernel_2d<KIND_KSPLIT, _Float16, B, S, W, D>(), kernel_2d<KIND_KSPLIT, __bf16, B, S, W, D>(),                   \
-   kernel_sel<KIND_KSPLIT, B, S, W, D>()}
+   BSG_SEL_FORMS(KIND_KSPLIT, B, S, W, D)}
 #define BSG_X(B, S, W, D)                                                                     \
   {KIND_XLDS, 16 * B, S, W, D, bsg_gemm_xl_kernel<_Float16, B, S, W, 1, D, false>,           \
    bsg_gemm_xl_kernel<__bf16, B, S, W, 1, D, false>, kernel_2d<KIND_XLDS, _Float16, B, S, W, D>(), \
-   kernel_2d<KIND_XLDS, __bf16, B, S, W, D>(), kernel_sel<KIND_XLDS, B, S, W, D>()}
+   kernel_2d<KIND_XLDS, __bf16, B, S, W, D>(), BSG_SEL_FORMS(KIND_XLDS, B, S, W, D)}
 #define BSG_Y(B, S, W, D)                                                                        \
   {KIND_XLDS_KH, 16 * B, S, W, D, bsg_gemm_xl_kernel<_Float16, B, S, W / 2, 2, D, false>,        \
    bsg_gemm_xl_kernel<__bf16, B, S, W / 2, 2, D, false>, kernel_2d<KIND_XLDS_KH, _Float16, B, S, W, D>(), \
-   kernel_2d<KIND_XLDS_KH, __bf16, B, S, W, D>(), kernel_sel<KIND_XLDS_KH, B, S, W, D>()}
+   kernel_2d<KIND_XLDS_KH, __bf16, B, S, W, D>(), BSG_SEL_FORMS(KIND_XLDS_KH, B, S, W, D)}
 #define BSG_V(B, S, W, D)                                                                               \
   {KIND_VT, 16 * B, S, W, D, bsg_gemm_vt_kernel<_Float16, B, S, W / 2, D>, bsg_gemm_vt_kernel<__bf16, B, S, W / 2, D>, \
-   nullptr, nullptr, kernel_sel<KIND_VT, B, S, W, D>()}
+   nullptr, nullptr, BSG_SEL_FORMS(KIND_VT, B, S, W, D)}
 #define BSG_V1(B, S, W, D)                                                                                \
   {KIND_VT1, 16 * B, S, W, D, bsg_gemm_vt_kernel<_Float16, B, S, W, D, 1>, bsg_gemm_vt_kernel<__bf16, B, S, W, D, 1>, \
-   nullptr, nullptr, kernel_sel<KIND_VT1, B, S, W, D>()}
+   nullptr, nullptr, BSG_SEL_FORMS(KIND_VT1, B, S, W, D)}
 #define BSG_V1X(B, S, W, D)                                                                                    \
   {KIND_VT1X, 16 * B, S, W, D, bsg_gemm_vtx_kernel<_Float16, B, S, W, D>, bsg_gemm_vtx_kernel<__bf16, B, S, W, D>, \
-   nullptr, nullptr, kernel_sel<KIND_VT1X, B, S, W, D>()}
+   nullptr, nullptr, BSG_SEL_FORMS(KIND_VT1X, B, S, W, D)}
 #define BSG_F(R, S, W, D)                                                                                 \
   {KIND_FMA, R, S, W, D, bsg_gemm_fma_kernel<_Float16, R, S, W, D, false>, bsg_gemm_fma_kernel<__bf16, R, S, W, D, false>, \
-   kernel_2d<KIND_FMA, _Float16, R, S, W, D>(), kernel_2d<KIND_FMA, __bf16, R, S, W, D>(), nullptr}
+   kernel_2d<KIND_FMA, _Float16, R, S, W, D>(), kernel_2d<KIND_FMA, __bf16, R, S, W, D>(), nullptr, nullptr, nullptr, nullptr}
 
 }  // namespace

@@ -197,6 +197,6 @@ __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
 
 #define BSG_R(B, S, RW, D)                                                                                       \
   {KIND_ROWS, 16 * B, S, 2 * RW, D, bsg_gemm_rows_kernel<_Float16, B, S, RW, D>, bsg_gemm_rows_kernel<__bf16, B, S, RW, D>, \
-   nullptr, nullptr, nullptr}
+   nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}
 
 }  // namespace
