@@ -941,14 +941,11 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   const int cnt = pend - pbeg;
 
   const int blk_bytes = p.npad * 128;
-  const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
   int xrow_off[BTT];
-  bool xrow_ok[BTT];
 #pragma unroll
   for (int bi = 0; bi < BTT; ++bi) {
     const int row = y0 + 16 * bi + (lane & 15);
-    xrow_ok[bi] = row < p.bt;
-    xrow_off[bi] = xrow_ok[bi] ? row * (int)p.ldx * 2 : 0;
+    xrow_off[bi] = row < p.bt ? row * (int)p.ldx * 2 : kOOB;
   }
   const int xcol = 8 * (lane >> 4);
   const int wcol = lane * 16 + (n0 >> 4) * 2048;
@@ -974,16 +971,17 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
       wd[s][0] = ld16_stream(wr, wcol + s * 2048);
       wd[s][1] = ld16_stream(wr, wcol + s * 2048 + 1024);
     }
+    // Skipped slots read through an empty resource and out-of-range lanes get the offset's top bit
+    // by arithmetic: with selects here every slot carried two branches.
+    const __amdgpu_buffer_rsrc_t xb = make_rsrc(p.x, ok ? p.x_bytes : 0);
     const int kb = (ok ? blk : 0) * 64 + xcol;
 #pragma unroll
-    for (int bi = 0; bi < BTT; ++bi) {
+    for (int bi = 0; bi < BTT; ++bi)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int col = kb + 32 * h;
-        const bool v = ok && xrow_ok[bi] && col < p.K;
-        xd[bi][h] = ld16(xr, v ? xrow_off[bi] + col * 2 : kOOB);
+        xd[bi][h] = ld16(xb, (xrow_off[bi] + col * 2) | (((p.K - 1 - col) >> 31) & kOOB));
       }
-    }
   };
 
   auto compute = [&](const u32x4 (&wd)[NSUB][2], const u32x4 (&xd)[BTT][2]) {
@@ -1110,17 +1108,14 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
   const int cnt = pend - pbeg;
 
   const int blk_bytes = p.npad * 128;
-  const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, p.x_bytes);
   // X fragments this wave brings in: f = w + j*WPG -> batch tile f/2, k-half f%2.
   int xrow_off[XPW];
-  bool xrow_ok[XPW];
   int xcol[XPW];
 #pragma unroll
   for (int j = 0; j < XPW; ++j) {
     const int f = w + j * WPG;
     const int row = y0 + 16 * (f >> 1) + (lane & 15);
-    xrow_ok[j] = f < XF && row < p.bt;
-    xrow_off[j] = xrow_ok[j] ? row * (int)p.ldx * 2 : 0;
+    xrow_off[j] = f < XF && row < p.bt ? row * (int)p.ldx * 2 : kOOB;
     xcol[j] = 32 * (f & 1) + 8 * (lane >> 4);
   }
   const int wcol = lane * 16 + ((n0 >> 4) + wc * NSUB) * 2048;
@@ -1145,12 +1140,13 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
     for (int s = 0; s < NSUB; ++s)
 #pragma unroll
       for (int hh = 0; hh < HPW; ++hh) wd[s][hh] = ld16_stream(wr, wcol + s * 2048 + (WK > 1 ? wk : hh) * 1024);
+    // as in kind 1: no select, so no branch, decides a lane's offset
+    const __amdgpu_buffer_rsrc_t xb = make_rsrc(p.x, ok ? p.x_bytes : 0);
     const int kb = (ok ? blk : 0) * 64;
 #pragma unroll
     for (int j = 0; j < XPW; ++j) {
       const int col = kb + xcol[j];
-      const bool v = ok && xrow_ok[j] && col < p.K;
-      xd[j] = ld16(xr, v ? xrow_off[j] + col * 2 : kOOB);
+      xd[j] = ld16(xb, (xrow_off[j] + col * 2) | (((p.K - 1 - col) >> 31) & kOOB));
     }
   };
 
