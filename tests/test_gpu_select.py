@@ -583,3 +583,67 @@ def test_energy_budget_inside_the_gemm(dev, dtype, bt, kdim, plan):
             ref = torch.empty_like(y)
             bsa.gemm_packed(xt, packed, n, s_ids[:c].contiguous(), ref, plan=p, num_active=c)
             assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+def test_select_prepared_call_rechecks_what_its_key_does_not_pin(dev):
+    """A repeated select_sparse_gemm call site takes a prepared launch.  What its key does not pin
+    must still be honoured: new x, out and id tensors, an in-place weight update (re-pack), an x 8
+    bytes past alignment and a non-contiguous out (refused, as by a first call), a released packed
+    weight, another stream, and a capture."""
+    from bsa_mi355x import runtime, select as sel
+
+    bt, k, n, kk = 2, 4096, 1040, 13
+    x, w_nk, _ = case(71, bt, k, n, 1, "normal")
+    wt = to_dev(w_nk, dev)
+
+    def run(xn, wn, xt=None, **kw):
+        xt = to_dev(xn, dev).view(bt, 1, k) if xt is None else xt
+        out = torch.full((bt, 1, n), float("nan"), dtype=torch.float16, device=dev)
+        idx, cnt = bsa.select_sparse_gemm(xt, wt, out, kk, cache_prefix="prep_sel", **kw)
+        torch.cuda.synchronize()
+        want = orc.select_topk_l1(xn, kk)
+        assert int(cnt.item()) == kk and np.array_equal(idx.cpu().numpy(), want)
+        assert_close(out.view(bt, n).float().cpu().numpy(), orc.gemm_ref(xn, wn, want), "prepared selection")
+
+    runtime.forget_prepared_calls()
+    run(x, w_nk)
+    assert len(sel._PREPARED_SELECT) == 1
+    x2, _, _ = case(72, bt, k, n, 1, "laplace")
+    run(x2, w_nk)
+    ids = torch.zeros(kk, dtype=torch.int32, device=dev)
+    run(x2, w_nk, idx_out=ids)
+    assert np.array_equal(ids.cpu().numpy(), orc.select_topk_l1(x2, kk))
+    with torch.no_grad():
+        wt.mul_(-0.5)
+    w2 = (w_nk.astype(np.float32) * -0.5).astype(np.float16)
+    run(x2, w2)
+    base = torch.empty(bt * k + 4, dtype=torch.float16, device=dev)
+    xo = base[4:].view(bt, 1, k)
+    xo.copy_(to_dev(x, dev).view(bt, 1, k))
+    with pytest.raises(bsa.BsgArgError):
+        run(x, w2, xt=xo)
+    run(x, w2)
+    big = torch.empty(bt, 2, n, dtype=torch.float16, device=dev)
+    with pytest.raises(ValueError):
+        bsa.select_sparse_gemm(to_dev(x, dev).view(bt, 1, k), wt, big[:, :1, :], kk, cache_prefix="prep_sel")
+    run(x, w2)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        run(x2, w2)
+    bsa.release_prepacked_weights("prep_sel")
+    assert not sel._PREPARED_SELECT
+    run(x2, w2)
+    xt = to_dev(x, dev).view(bt, 1, k)
+    out = torch.zeros(bt, 1, n, dtype=torch.float16, device=dev)
+    cnt = torch.zeros(1, dtype=torch.int32, device=dev)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        bsa.select_sparse_gemm(xt, wt, out, kk, cache_prefix="prep_sel", idx_out=ids, count_out=cnt)
+    for xn in (x, x2, x):
+        xt.copy_(to_dev(xn, dev).view(bt, 1, k))
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        want = orc.select_topk_l1(xn, kk)
+        assert np.array_equal(ids.cpu().numpy(), want)
+        assert_close(out.view(bt, n).float().cpu().numpy(), orc.gemm_ref(xn, w2, want), "captured")
