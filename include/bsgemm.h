@@ -53,7 +53,7 @@ enum bsg_status {
  *   cols_per_wave   : output columns per wavefront (kinds 1-4: 16, 32, 64 or 128); kinds 5-8:
  *                     the most columns one work-group may take (16 x its most subtiles)
  *   waves_per_group : wavefronts per work-group: 1, 2, 4 or 8
- *   depth           : K-blocks whose loads each wave keeps in flight: 1, 2, 4 or 8
+ *   depth           : K-blocks whose loads each wave keeps in flight: 1, 2, 3, 4 or 8
  *   rows_per_group  : batch rows per work-group (16, 32 or 64; 1, 2, 4 or 8 for kind 3; 128 for
  *                     kind 8); bt above it adds row groups
  *   kind            : the kernel family.

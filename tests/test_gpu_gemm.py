@@ -670,3 +670,46 @@ def test_variable_width_column_groups(dev, bt, k, n, na):
         torch.cuda.synchronize()
         assert_close(dense.float().cpu().numpy(), ref_dense, f"kind {kind} dense")
         assert_close(bout.float().cpu().numpy(), ref, f"kind {kind} bitmap")
+
+
+@pytest.mark.parametrize("bt,k,n,na", [(1, 2048, 2048, 16), (16, 1000, 8200, 9), (24, 1024, 13824, 12),
+                                       (33, 512, 20000, 8), (64, 640, 16384, 10), (48, 4096, 4096, 64),
+                                       (40, 8192, 4096, 100)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_plans_by_size(dev, bt, k, n, na, dtype):
+    """Shapes the table does not hold, under capture (no first-call tuning) and through a selection:
+    the plan by size, list and bitmap (every sparsity from one block to all), against the oracle."""
+    from bsa_mi355x import tuning
+
+    x, w_nk, idx = case(500 + bt, bt, k, n, na, "normal")
+    xt, wt = torch.from_numpy(x).to(dtype), torch.from_numpy(w_nk).to(dtype)
+    xo, wo = xt.float().numpy(), wt.float().numpy()
+    xt = xt.to(dev)
+    packed = bsa.pack_weight(wt.to(dev))
+    nblk = orc.nblk_of(k)
+    want = tuning.sized_plan(bt, n, na)
+    got = bsa.resolve_plan(bt, n, nblk, na, dev)
+    if (n, nblk) not in tuning._INDEX:
+        assert want is None or got.as_tuple() == want.as_tuple()
+    rng = np.random.default_rng(bt)
+    for keep in sorted({1, na, nblk}):
+        ids = np.sort(rng.choice(nblk, keep, replace=False)).astype(np.int32)
+        ref = orc.gemm_ref64(xo, wo, ids)
+        bm = torch.zeros(nblk, dtype=torch.uint8, device=dev)
+        bm[torch.from_numpy(ids).long().to(dev)] = 7
+        outs = [torch.full((bt, n), float("nan"), dtype=dtype, device=dev) for _ in range(2)]
+        print(f"sized bt={bt} K={k} N={n} keep={keep} {dtype}", flush=True)
+        bsa.gemm_packed(xt, packed, n, to_dev(ids, dev), outs[0], plan=got)
+        bsa.gemm_packed(xt, packed, n, None, outs[1], bitmap=bm, plan=got)
+        for o in outs:
+            err = np.linalg.norm(o.float().cpu().numpy() - ref) / np.linalg.norm(ref)
+            # the output's rounding alone: 2^-11 (fp16) or 2^-8 (bf16) of a value at most
+            assert err <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), err
+    from bsa_mi355x.select import select_gemm_rule_packed
+    y = torch.empty(bt, n, dtype=dtype, device=dev)
+    ids, cnt, _ = select_gemm_rule_packed(xt, packed, n, na, y, score="energy")
+    c = int(cnt.item())
+    kept, _, _ = orc.select_scored_ref(xo, na, "energy")
+    assert np.array_equal(ids[:c].cpu().numpy(), kept)
+    ref = orc.gemm_ref64(xo, wo, kept)
+    assert np.linalg.norm(y.float().cpu().numpy() - ref) <= 2.0 ** -8 * np.linalg.norm(ref)

@@ -358,3 +358,18 @@ def test_many_rows_plans_resolve_unchanged():
             q = bsa.Plan(*p.as_tuple())
             assert bsa.load().bsg_plan_resolve(bt, n, 64, 31, 256, ctypes.byref(q)) == 0, (bt, n, p.as_tuple())
             assert q.as_tuple() == p.as_tuple() and p.rows_per_group >= 64
+
+
+def test_sized_plans_resolve_unchanged():
+    """Every plan tuning.sized_plan gives names a compiled tile that the library takes as it is, at
+    every width and batch; None only for long lists over few columns past 16 rows."""
+    for bt in (1, 2, 7, 16, 17, 32, 33, 64, 65, 300):
+        for n in (1, 16, 100, 1000, 2048, 4096, 4097, 8192, 8193, 12288, 12289, 16384, 16385, 24576, 40000):
+            for na in (0, 1, 31, 86, 512):
+                p = tuning.sized_plan(bt, n, na)
+                if p is None:
+                    assert 16 < bt <= 64 and n <= 4096 and na * -(-n // 16) > 20000
+                    continue
+                q = bsa.Plan(*p.as_tuple())
+                assert bsa.load().bsg_plan_resolve(bt, n, 512, na, 256, ctypes.byref(q)) == 0, (bt, n, p.as_tuple())
+                assert q.as_tuple() == p.as_tuple()

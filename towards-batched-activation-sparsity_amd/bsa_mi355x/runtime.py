@@ -209,18 +209,18 @@ _RESOLVED: dict = {}
 
 
 def resolve_plan(bt: int, n: int, nblk: int, na: int, device: torch.device, plan: Optional[Plan] = None,
-                 dense: bool = False, lookup_plan: bool = True, select: bool = False) -> Plan:
+                 dense: bool = False, lookup_plan: bool = True, select: bool = False, sized: bool = True) -> Plan:
     """Resolve a (partial) plan for a problem.  With no plan (or an all-zero one) the tuned
     table (tuning.lookup; select=True: the entries timed as selection + GEMM first) is consulted
-    first (past 64 rows, tuning.many_rows_plan); remaining zero fields are filled by the library's heuristics; tile fields that name a
+    first, then (sized) the plan by size, tuning.sized_plan; remaining zero fields are filled by the library's heuristics; tile fields that name a
     kernel that is not instantiated fall back to automatic (the split-K factor is kept)."""
     lib = load()
     if lookup_plan and (plan is None or not any(plan.as_tuple())):
         from . import tuning
 
         tuned = tuning.lookup(bt, n, nblk, na, dense=dense, select=select)
-        if tuned is None and bt > 64:
-            tuned = tuning.many_rows_plan(bt, n)
+        if tuned is None and sized:
+            tuned = tuning.sized_plan(bt, n, na)
         if tuned is not None:
             plan = tuned
     req = plan.as_tuple() if plan is not None else (0, 0, 0, 0, 0, 0)
@@ -711,7 +711,7 @@ def kernel_tiles() -> Sequence[tuple]:
         for rows in ((1, 2, 4, 8) if kind == 3 else (128,) if kind == 8 else (16, 32, 64)):
             for cols in ((16, 32, 48, 64, 96) if kind >= 5 else (16, 32, 64, 128)):
                 for waves in (1, 2, 4, 8):
-                    for depth in (1, 2, 4, 8):
+                    for depth in (1, 2, 3, 4, 8):
                         p = Plan(1, cols, waves, depth, rows, kind)
                         if load().bsg_plan_resolve(rows, cols, 1, 1, 1, ctypes_byref(p)) == _lib.BSG_OK:
                             out.append((kind, rows, cols, waves, depth))

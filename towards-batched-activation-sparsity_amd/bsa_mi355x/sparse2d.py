@@ -56,8 +56,9 @@ def plan_2d(bt: int, n_dim: int, nn: int, nblk: int, na: int, device: torch.devi
     at most 4 for 32- and 64-row tiles (their partials are large) and 8 otherwise, measured on
     down_proj B=16 and B=64 with 16-64 of 64 output blocks."""
     explicit = plan is not None and any(plan.as_tuple())
-    # the automatic tile is that of up to 64 rows: larger 1-D batches run tiles with no 2-D form
-    pl = resolve_plan(bt if explicit else min(int(bt), 64), n_dim, nblk, na, device, plan, dense=dense)
+    # the automatic tile is that of up to 64 rows, tabulated or the library's: the plans by size and
+    # for larger batches run tiles with no 2-D form
+    pl = resolve_plan(bt if explicit else min(int(bt), 64), n_dim, nblk, na, device, plan, dense=dense, sized=False)
     if pl.kind >= 5:
         # variable-width column groups have no 2-D instantiation: the 16-column list-splitting
         # tile of the same rows instead

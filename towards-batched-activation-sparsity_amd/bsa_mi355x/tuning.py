@@ -65,6 +65,32 @@ def many_rows_plan(bt: int, n: int) -> Plan:
     return Plan(2, 32, 8, 4, 64, 4)
 
 
+def sized_plan(bt: int, n: int, na: int) -> Optional[Plan]:
+    """Plan by size for a problem without a tuned one (a selection + GEMM, or a capture, of a shape
+    the table does not hold): variable-width column groups of as many 16-column subtiles as one
+    compute unit gets, which fill the chip at any width, where the library's heuristic rounds to 16
+    or 64 columns and splits the list.  Up to 16 rows kinds 6 and 5, to 32 two 16-row groups or
+    kinds 7 and 5, to 64 kind 7.  Measured beside the heuristic, GEMM / selection + GEMM, us:
+    N=2048 K=2048 16 blocks, 5 rows 3.6 against 5.5 / 7.4 against 11.9, 64 rows 4.9, 9.1 / 8.1, 12.0;
+    N=13824 K=5120 32 blocks, 16 rows 13.1, 15.9 / 17.2, 21.3, 64 rows 16.0, 21.8 / 20.5, 26.5.
+    None (the heuristic) for long lists over few columns past 16 rows, where its split-K wins:
+    N=4096, 96 blocks, 24 / 48 rows 13.3 / 16.1 against 15.9 / 18.1, while N=3072, 89 blocks, takes
+    13.6 / 16.0 here against 14.2 / 18.8."""
+    if bt > 64:
+        return many_rows_plan(bt, n)
+    tiles = -(-int(n) // 16)
+    s = -(-tiles // _CUS)
+    cols = 16 * (s if s <= 4 else 6)
+    if s == 1 and bt > 16 and na * tiles > 20000:
+        return None
+    if bt <= 16:
+        return Plan(1, cols, 4, 4, 16, 6 if s == 1 else 5)
+    if bt <= 32:
+        return Plan(1, 32, 4, 4, 16, 5) if s == 1 else Plan(1, cols, 4, 2, 32, 7) if s <= 4 else \
+            Plan(1, 96, 4, 4, 32, 5)
+    return Plan(1, 32, 4, 2, 32, 7) if s == 1 else Plan(1, cols, 4, 2, 64, 7) if s <= 4 else Plan(1, 96, 4, 3, 64, 7)
+
+
 # ---------------------------------------------------------------------------------------
 # Run-time lookup
 

@@ -747,7 +747,7 @@ __device__ __forceinline__ int list_entry_of_thread(const GemmParams& p) {
 // self-scored form), in the selection forms of KernelEntry, which are launched in those modes only;
 // without the list, bitmap and dense branches beside it the selection + GEMM calls take 2-4% less.
 template <int NT, int SEL = SEL_NONE, bool SELF_SCORE = false>
-__device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids, int* s_scan, int first) {
+__device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids, int first) {
   const int tid = threadIdx.x;
   int na = 0;
   if constexpr (SEL == SEL_TOPK) {
@@ -777,16 +777,26 @@ __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids,
     else
       for (int i = tid; i < na; i += NT) s_ids[i] = p.idx[i];
   } else if (p.mode == MODE_BITMAP) {
-    const int per = (p.nbm + NT - 1) / NT;
-    const int beg = tid * per < p.nbm ? tid * per : p.nbm;
-    const int end = beg + per < p.nbm ? beg + per : p.nbm;
-    int c = 0;
-    for (int i = beg; i < end; ++i) c += p.bitmap[i] != 0;
-    int total = 0;
-    int o = wg_exclusive_scan<NT>(c, s_scan, &total);
-    for (int i = beg; i < end; ++i)
-      if (p.bitmap[i] != 0) s_ids[o++] = i;
-    na = total;
+    // Every wave ballots the flags of each 64-block group and keeps the running count, so a
+    // block's position needs no scan over the work-group; wave g % W writes group g.  The flags of
+    // U groups are requested together.
+    constexpr int U = 8, W = NT / 64;
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int g0 = 0; 64 * g0 < p.nbm; g0 += U) {
+      uint8_t f[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = 64 * (g0 + u) + lane;
+        f[u] = i < p.nbm ? p.bitmap[i] : (uint8_t)0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint64_t m = __ballot(f[u] != 0);
+        if ((g0 + u) % W == w && f[u] != 0)
+          s_ids[na + __popcll(m & ((1ull << lane) - 1ull))] = 64 * (g0 + u) + lane;
+        na += __popcll(m);
+      }
+    }
   } else {
     na = p.nblk;
     for (int i = tid; i < na; i += NT) s_ids[i] = i;
@@ -914,7 +924,7 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   constexpr int IDS_BYTES = BSG_MAX_NBLK * 4;
   // The block list (main loop) and the wave-reduction buffer (epilogue) share LDS.
   __shared__ __attribute__((aligned(16))) char s_mem[RED_BYTES > IDS_BYTES ? RED_BYTES : IDS_BYTES];
-  __shared__ int s_misc[WPG + 2];
+  __shared__ int s_last;  // split-K: this work-group reduces its tile
   int* const s_ids = (int*)s_mem;
   f32x4* const s_red = (f32x4*)s_mem;
 
@@ -930,7 +940,7 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, first);
   BSG_TL(1);
 
   // This wave's contiguous slice [pbeg, pend) of the list.
@@ -1059,8 +1069,8 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   }
 
   BSG_TL(4);
-  if (S > 1) splitk_finish<T, BTT, NSUB, NSUB, F>(p, tile_lin, y0, n0y, sk, 0, w == 0, acc, &s_misc[WPG]);
-  BSG_TL_END(p, S == 1 || s_misc[WPG] != 0);
+  if (S > 1) splitk_finish<T, BTT, NSUB, NSUB, F>(p, tile_lin, y0, n0y, sk, 0, w == 0, acc, &s_last);
+  BSG_TL_END(p, S == 1 || s_last != 0);
 }
 
 // Kinds 2 and 4 ("xlds"): one work-group = BTT*16 batch rows x WC*NSUB*16 columns; its waves
@@ -1083,7 +1093,7 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
   __shared__ __attribute__((aligned(16))) int s_ids[BSG_MAX_NBLK];
   __shared__ __attribute__((aligned(16))) u32x4 s_x[2][XF][64];
   __shared__ __attribute__((aligned(16))) f32x4 s_red[WK > 1 ? WC * BTT * NSUB : 1][64];
-  __shared__ int s_misc[WPG + 2];
+  __shared__ int s_last;  // split-K: this work-group reduces its tile
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1099,7 +1109,7 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, first);
   BSG_TL(1);
 
   // The work-group's contiguous slice of the list (all its waves walk it together).
@@ -1229,8 +1239,8 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
       }
   }
   BSG_TL(4);
-  if (S > 1) splitk_finish<T, BTT, NSUB, CS, FT>(p, tile_lin, y0, n0y, sk, wc, wk == 0, acc, &s_misc[WPG]);
-  BSG_TL_END(p, S == 1 || s_misc[WPG] != 0);
+  if (S > 1) splitk_finish<T, BTT, NSUB, CS, FT>(p, tile_lin, y0, n0y, sk, wc, wk == 0, acc, &s_last);
+  BSG_TL_END(p, S == 1 || s_last != 0);
 }
 
 // Kind 3 ("fma", batch tiles of 1-8 rows): the contraction is too thin for MFMA, so each lane
@@ -1250,7 +1260,6 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_fma_kernel(GemmParams p) {
   constexpr int XI = BSG_FMA_X_LOADS;  // staging loads per wave (host guarantees enough)
   __shared__ __attribute__((aligned(16))) int s_ids[BSG_MAX_NBLK];
   __shared__ float s_red[WPG > 1 ? WPG - 1 : 1][NSUB * BT][16];
-  __shared__ int s_misc[WPG + 2];
   extern __shared__ __attribute__((aligned(16))) u32x4 s_xs[];  // [na][BT][2][4]
 
   const int lane = threadIdx.x & 63;
@@ -1263,7 +1272,7 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_fma_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT>(p, s_ids, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * w) / WPG);
   const int pend = (int)(((int64_t)na * (w + 1)) / WPG);
@@ -1458,7 +1467,6 @@ __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p)
   constexpr int HP = 3 - KH;  // halves per wave
   __shared__ __attribute__((aligned(16))) int s_ids[BSG_MAX_NBLK];
   __shared__ __attribute__((aligned(16))) f32x4 s_red[NW][F][64];
-  __shared__ int s_misc[NW + 2];
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1473,7 +1481,7 @@ __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p)
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * b) / WB);
   const int pend = (int)(((int64_t)na * (b + 1)) / WB);
@@ -1597,7 +1605,6 @@ __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   static_assert(F <= DEPTH * SLOT, "the wave reduction reuses the wave's own activation slots");
   __shared__ __attribute__((aligned(16))) int s_ids[BSG_MAX_NBLK];
   __shared__ __attribute__((aligned(16))) u32x4 s_x[WB * DEPTH * SLOT][64];
-  __shared__ int s_misc[WB + 2];
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the wave's block slice
@@ -1610,7 +1617,7 @@ __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, s_misc, first);
+  const int na = stage_block_list<NT, SEL, SEL == SEL_TOPK && BTT == 1 && std::is_same<T, _Float16>::value>(p, s_ids, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * w) / WB);
   const int pend = (int)(((int64_t)na * (w + 1)) / WB);

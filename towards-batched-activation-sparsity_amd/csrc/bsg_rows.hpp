@@ -40,7 +40,6 @@ __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
   constexpr int RF = RT * NSUB;                   // output fragments per row part
   static_assert(RF <= PIECES && RW <= DEPTH, "each row part's halves meet in a stage of their own");
   __shared__ __attribute__((aligned(16))) int s_ids[BSG_MAX_NBLK];
-  __shared__ int s_misc[NW + 2];
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -57,7 +56,7 @@ __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT>(p, s_ids, s_misc, list_entry_of_thread(p));
+  const int na = stage_block_list<NT>(p, s_ids, list_entry_of_thread(p));
   BSG_TL(1);
 
   const int blk_bytes = p.npad * 128;

@@ -12,6 +12,10 @@ const KernelEntry kEntries[] = {
     // waves (eight: two per SIMD)
     BSG_V1X(4, 3, 4, 2), BSG_V1X(4, 3, 4, 3), BSG_V1X(4, 3, 4, 4), BSG_V1X(4, 3, 2, 4), BSG_V1X(4, 2, 4, 2),
     BSG_V1X(4, 2, 4, 4), BSG_V1X(4, 3, 8, 2), BSG_V1X(4, 2, 8, 2),
+    // 256 groups of up to 4 subtiles at N = 12304 to 16384 (64 rows, N = 16000, 31 blocks: 15.5 us,
+    // the best tile before 17.8; N = 13827, K = 5000, 32 blocks: 15.7 / 16.5), and of up to 6 to
+    // N = 24576 (N = 20000, K = 5120, 40 blocks: 23.6 / 24.6)
+    BSG_V1X(4, 4, 4, 2), BSG_V1X(4, 6, 4, 3),
     // 32 rows (one row group of a 32-row batch, or half of a 64-row one)
     BSG_V1X(2, 2, 4, 2), BSG_V1X(2, 3, 4, 2), BSG_V1X(2, 2, 4, 4), BSG_V1X(2, 3, 4, 4), BSG_V1X(2, 4, 4, 2),
     BSG_V1X(2, 2, 8, 2), BSG_V1X(2, 3, 8, 2),
