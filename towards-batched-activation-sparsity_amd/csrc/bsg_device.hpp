@@ -34,7 +34,7 @@ struct GemmParams {
     int32_t nbm;        // MODE_BITMAP: entries of the bitmap
     float energy_keep;  // MODE_TOPK_BUDGET: the energy fraction to keep (0: none)
   };
-  int32_t na, mode, split_k, n_tiles, x_bytes, y_fast;
+  int32_t na, mode, split_k, n_tiles, x_bytes;
   // MODE_TOPK: exact-L1 block scores (na = k), whether they fit the unique-key order, and where
   // work-group (0, 0) publishes the kept list and its count (null: not published)
   const uint64_t* scores;
@@ -93,6 +93,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));  // 8 bytes at 2-byte alignment
 
 constexpr int kOOB = (int)0x80000000u;  // buffer offset beyond any num_records we build
 constexpr int kRsrcWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
@@ -821,18 +822,17 @@ __device__ __forceinline__ void store_y(const GemmParams& p, int y0, int n0, int
   const int n = n0 + 16 * cs + 4 * (lane >> 4);
   if (b >= p.bt) return;
   uint16_t* yrow = (uint16_t*)p.y + (size_t)b * (size_t)p.ldy;
-  if (p.y_fast) {
-    if (n < p.ny) {
-      u32x2 pk;
-      pk.x = (uint32_t)Elem<T>::bits(v.x) | ((uint32_t)Elem<T>::bits(v.y) << 16);
-      pk.y = (uint32_t)Elem<T>::bits(v.z) | ((uint32_t)Elem<T>::bits(v.w) << 16);
-      *(u32x2*)(yrow + n) = pk;
-    }
+  // One 8-byte store of the lane's 4 columns, whatever the row's alignment (global stores need only
+  // their elements'); the last columns of an N that is not a multiple of 4 go one by one.
+  if (n + 4 <= p.ny) {
+    u32x2_a2 pk;
+    pk.x = (uint32_t)Elem<T>::bits(v.x) | ((uint32_t)Elem<T>::bits(v.y) << 16);
+    pk.y = (uint32_t)Elem<T>::bits(v.z) | ((uint32_t)Elem<T>::bits(v.w) << 16);
+    *(u32x2_a2*)(yrow + n) = pk;
   } else {
     if (n + 0 < p.ny) yrow[n + 0] = Elem<T>::bits(v.x);
     if (n + 1 < p.ny) yrow[n + 1] = Elem<T>::bits(v.y);
     if (n + 2 < p.ny) yrow[n + 2] = Elem<T>::bits(v.z);
-    if (n + 3 < p.ny) yrow[n + 3] = Elem<T>::bits(v.w);
   }
 }
 

@@ -821,7 +821,6 @@ int launch_gemm(int mode, const void* x, int64_t ldx, int64_t bt, int64_t K, con
   p.n_tiles = (int32_t)n_tiles;
   p.x_bytes = (int32_t)(((bt - 1) * ldx + K) * 2);
   p.ny = (int32_t)y_cols;
-  p.y_fast = (y_cols % 4 == 0) && (ldy % 4 == 0) && (((uintptr_t)y & 7u) == 0);
   p.scores = ex.scores;
   p.idx_out = ex.idx_out;
   p.na_out = ex.na_out;
