@@ -54,7 +54,14 @@ def plan_2d(bt: int, n_dim: int, nn: int, nblk: int, na: int, device: torch.devi
     full N (the tuned table), or the library's when that one is wider than 64 columns, and the
     split-K factor fills the chip without a partial second round: floor(CUs / work-groups),
     at most 4 for 32- and 64-row tiles (their partials are large) and 8 otherwise, measured on
-    down_proj B=16 and B=64 with 16-64 of 64 output blocks."""
+    down_proj B=16 and B=64 with 16-64 of 64 output blocks.  Up to 8 rows no split pays for its
+    hand-off: four list-splitting waves on 16 columns (K=N=4096, 32 x 20 blocks, 2 rows 6.3 us against
+    7.8 with split-K 3; K=11008, 60 x 32 blocks 8.7 / 9.8; N=22016, 16 x 300 blocks, 1 row 11.7 / 12.7).
+    At 9-16 rows the 16-column tile widens while its tiles outnumber the compute units (K=4096
+    N=11008, 32 x 86 blocks 10.2 / 11.8, 32 x 170 blocks 13.5 / 14.5; not past one 64-column tile per
+    unit: N=22016, 30 x 300 blocks 21.8 / 20.3), and a split leaves each wave at
+    least 5 blocks (K=N=2048, 16 x 16 blocks 5.3 / 7.0; 64 x 24 blocks keep split-K 2, 9.7 against
+    10.4 without)."""
     explicit = plan is not None and any(plan.as_tuple())
     # the automatic tile is that of up to 64 rows, tabulated or the library's: the plans by size and
     # for larger batches run tiles with no 2-D form
@@ -74,10 +81,19 @@ def plan_2d(bt: int, n_dim: int, nn: int, nblk: int, na: int, device: torch.devi
                           lookup_plan=False)
     if explicit and plan.split_k:
         return pl
+    if not explicit and int(bt) <= 8:
+        return Plan(1, 16, 4, 4, 16, 1)
+    cols = pl.cols_per_wave
+    if not explicit and pl.kind == 1 and pl.rows_per_group == 16 and nn <= _cu_count(device):
+        while cols < BLOCK_N_OUT and max(1, nn) * (BLOCK_N_OUT // cols) > _cu_count(device):
+            cols *= 2
+        if cols > pl.cols_per_wave:
+            pl = Plan(1, cols, 4 if cols == BLOCK_N_OUT else 2, 4, 16, 1)
     groups = max(1, nn) * (BLOCK_N_OUT // pl.group_cols()) * (-(-int(bt) // pl.rows_per_group))
     cap = 4 if pl.rows_per_group >= 32 else 8
     splitters = pl.waves_per_group if pl.kind == 1 else 1
-    sk = max(1, min(cap, _cu_count(device) // groups, max(1, int(na) // (2 * splitters))))
+    per_wave = 5 if pl.rows_per_group == 16 and not explicit else 2
+    sk = max(1, min(cap, _cu_count(device) // groups, max(1, int(na) // (per_wave * splitters))))
     if pl.kind == 3:
         sk = 1
     return Plan(sk, pl.cols_per_wave, pl.waves_per_group, pl.depth, pl.rows_per_group, pl.kind)
