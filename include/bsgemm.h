@@ -209,7 +209,9 @@ int bsg_gemm_2d(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* w
  *   sort_active  : non-zero sorts the K-block list while it is staged (num_active <= BSG_MAX_NBLK / 2)
  *   n_sorted_out : non-null (device, room for num_n) when n_blocks holds num_n_list ids in any order
  *                  (at most 512, else BSG_ERR_UNSUPPORTED): the num_n lowest are computed and
- *                  written there ascending; null takes n_blocks[num_n] as it is.
+ *                  written there ascending; null takes n_blocks[num_n] as it is.  It must not
+ *                  overlap n_blocks[num_n_list] or active_blocks[num_active] (BSG_ERR_ARG): the
+ *                  lists are still being read while it is written.
  * With num_n = 0 nothing is written.  The result is bsg_gemm_2d on the sorted lists, bit for bit. */
 int bsg_gemm_2d_sorted(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
                        const int32_t* active_blocks, int32_t num_active, int sort_active,

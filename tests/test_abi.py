@@ -233,6 +233,30 @@ def test_2d_entry_points_reject_bad_arguments_without_launching():
     assert lib.bsg_nmask_blocks(None, 64, FAKE, FAKE, None) == _lib.BSG_ERR_ARG
 
 
+def test_2d_sorted_output_list_may_not_overlap_the_lists():
+    """bsg_gemm_2d_sorted writes the sorted ids while other work-groups still read both lists, so
+    the ranges may share no entry.  The plan needs a workspace that no call here has, so a call
+    that passes the range check ends there and nothing launches."""
+    lib = bsa.load()
+    p = _lib.Plan(2, 16, 2, 4, 16, 1)
+    nb, kb = FAKE, FAKE + (1 << 20)  # 8 output blocks, 10 K-blocks
+
+    def call(out, nn=3, idx=kb, na=10, sort=1):
+        return lib.bsg_gemm_2d_sorted(FAKE, 4096, 16, 4096, FAKE, 4096, idx, na, sort, nb, 8, nn, out, 0, FAKE, 4096, 0,
+                                      None, 0, ctypes.byref(p), None)
+
+    for start, count in ((nb, 8), (kb, 10)):
+        for out in (start, start + 4, start + 4 * (count - 1), start - 8):  # 3 ids of 4 bytes each
+            for sort in (0, 1):
+                assert call(out, sort=sort) == _lib.BSG_ERR_ARG, (hex(out), sort)
+                assert "overlap" in _lib.last_error()
+        for out in (start + 4 * count, start - 12):  # right behind and right in front
+            assert call(out) == _lib.BSG_ERR_WORKSPACE, hex(out)
+    assert call(None) == _lib.BSG_ERR_WORKSPACE
+    assert call(kb, idx=None, na=0) == _lib.BSG_ERR_WORKSPACE  # every K-block: no list to overlap
+    assert call(nb, nn=0) == _lib.BSG_OK                       # nothing is written
+
+
 def test_bitmap_and_select_reject_bad_arguments():
     lib = bsa.load()
     p = _lib.Plan(1, 32, 4, 4, 16, 1)

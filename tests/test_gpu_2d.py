@@ -300,3 +300,20 @@ def test_2d_entry_points_past_the_in_kernel_sort(dev):
     _, blocks = s2d._prepacked_block_sparse_gemm_2d_from_active_blocks(x, w, kb, nb[:9], out, active_n_blocks_limit=0,
                                                                        cache_prefix="long2d")
     assert torch.equal(blocks, nb[:9].sort()[0]) and not torch.any(out)
+
+
+def test_2d_sorted_output_list_needs_memory_of_its_own(dev):
+    """gemm_2d_packed refuses an n_sorted_out that shares entries with either list it reads."""
+    bt, kdim, n = 4, 640, 1024
+    x, w_nk, _ = case(8, bt, kdim, n, 1, "normal")
+    packed, xt = bsa.pack_weight(to_dev(w_nk, dev)), to_dev(x, dev)
+    y = torch.full((bt, n), SENTINEL, dtype=torch.float16, device=dev)
+    buf = torch.tensor([9, 3, 5, 1, 0, 0], dtype=torch.int32, device=dev)
+    for lists in ((buf[:4], buf[:4]), (buf[:4], buf[3:6]), (buf[2:5], buf[:3])):
+        with pytest.raises(ValueError):
+            s2d.gemm_2d_packed(xt, packed, n, None, lists[0], y, num_n=3, n_sorted_out=lists[1])
+    with pytest.raises(ValueError):
+        s2d.gemm_2d_packed(xt, packed, n, buf[:3], torch.tensor([2, 1], dtype=torch.int32, device=dev), y,
+                           sort_active=True, n_sorted_out=buf[2:4])
+    torch.cuda.synchronize()
+    assert bool((y == SENTINEL).all()) and buf.tolist() == [9, 3, 5, 1, 0, 0]

@@ -112,8 +112,8 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
     64-column output blocks (ascending), host length `num_n`, optional device count
     `num_n_dev`.  sort_active: the GEMM sorts the K-block list ascending itself (at most
     MAX_NBLK // 2 entries); n_sorted_out (int32, at least num_n): n_blocks is in any order (at most
-    SORT_N_MAX entries) and the GEMM takes its num_n lowest, writing them there ascending (both
-    with host counts only).  compact=False: y2d is [bt, N] and only the active blocks' columns are
+    SORT_N_MAX entries) and the GEMM takes its num_n lowest, writing them there ascending, while the
+    lists are still read: memory of its own (both with host counts only).  compact=False: y2d is [bt, N] and only the active blocks' columns are
     written; compact=True: y2d is [bt, num_n * 64], list entry i at columns 64i.."""
     lib = load()
     dev = _require_cuda(x2d, packed, y2d)
@@ -137,9 +137,8 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
         raise ValueError("in-kernel sorting takes host counts")
     nb = _int32_dev(n_blocks, dev)
     if n_sorted_out is not None and (n_sorted_out.dtype != torch.int32 or n_sorted_out.device != dev
-                                     or not n_sorted_out.is_contiguous() or int(n_sorted_out.numel()) < nn
-                                     or n_sorted_out.data_ptr() == nb.data_ptr()):
-        raise ValueError(f"n_sorted_out must be another int32 tensor of at least {nn} entries on {dev}")
+                                     or not n_sorted_out.is_contiguous() or int(n_sorted_out.numel()) < nn):
+        raise ValueError(f"n_sorted_out must be a contiguous int32 tensor of at least {nn} entries on {dev}")
     if active_blocks is not None:
         ab = _int32_dev(active_blocks, dev)
         na = int(ab.numel() if num_active is None else num_active)

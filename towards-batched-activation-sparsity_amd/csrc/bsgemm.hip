@@ -993,6 +993,12 @@ int bsg_gemm_dense(const void* x, int64_t ldx, int64_t bt, int64_t K, const void
                      ws_bytes, plan, stream);
 }
 
+// Whether int32 ranges a[na] and b[nb] share an address (a null or empty range shares none).
+static bool ranges_overlap(const int32_t* a, int64_t na, const int32_t* b, int64_t nb) {
+  const uintptr_t pa = (uintptr_t)a, pb = (uintptr_t)b;
+  return a != nullptr && b != nullptr && na > 0 && nb > 0 && pa < pb + 4 * (uintptr_t)nb && pb < pa + 4 * (uintptr_t)na;
+}
+
 static int gemm_2d_run(const void* x, int64_t ldx, int64_t bt, int64_t K, const void* wp, int64_t N,
                        const int32_t* active_blocks, int32_t num_active, const int32_t* num_active_dev,
                        int32_t num_n, void* y, int64_t ldy, int dtype, void* ws, int64_t ws_bytes,
@@ -1030,6 +1036,11 @@ int bsg_gemm_2d_sorted(const void* x, int64_t ldx, int64_t bt, int64_t K, const 
     return fail(num_n_list < num_n ? BSG_ERR_ARG : BSG_ERR_UNSUPPORTED,
                 "2-D in-kernel sort: a list of %d output blocks, %d taken (at most %d)", num_n_list, num_n,
                 BSG_2D_SORT_MAX);
+  // one work-group writes the sorted ids while the others still read both lists
+  if (n_sorted_out != nullptr && num_n > 0 &&
+      (ranges_overlap(n_sorted_out, num_n, n_blocks, num_n_list) ||
+       ranges_overlap(n_sorted_out, num_n, active_blocks, num_active)))
+    return fail(BSG_ERR_ARG, "2-D in-kernel sort: n_sorted_out overlaps n_blocks or active_blocks");
   LaunchExtras ex;
   ex.nidx = n_blocks;
   ex.nn = num_n;
