@@ -373,3 +373,28 @@ def test_sized_plans_resolve_unchanged():
                 q = bsa.Plan(*p.as_tuple())
                 assert bsa.load().bsg_plan_resolve(bt, n, 512, na, 256, ctypes.byref(q)) == 0, (bt, n, p.as_tuple())
                 assert q.as_tuple() == p.as_tuple()
+
+
+def test_2d_plans_split_long_lists_over_few_output_blocks(monkeypatch):
+    """Up to 8 rows a 2-D launch with few output blocks splits a long list over the idle compute
+    units; short lists and many output blocks stay unsplit, and no split starts more work-groups
+    than there are units or leaves a wave fewer than 4 blocks."""
+    import torch
+
+    from bsa_mi355x import runtime, sparse2d
+
+    for cus in (256, 64):
+        monkeypatch.setattr(runtime, "_cu_count", lambda d: cus)
+        monkeypatch.setattr(sparse2d, "_cu_count", lambda d: cus)
+        dev = torch.device("cuda", 0)
+        for bt in (1, 4, 8):
+            for nn in (1, 3, 5, 8, 16, 24, 32, 64):
+                for na in (0, 1, 4, 8, 16, 32, 64, 128, 172, 192):
+                    p = sparse2d.plan_2d(bt, 4096, nn, 192, na, dev)
+                    assert p.as_tuple()[1:] == (16, 4 if na >= 8 else 2, 4, 16, 1), p.as_tuple()
+                    groups = 4 * nn
+                    assert p.split_k == 1 or (groups * p.split_k <= cus and na >= 16 * p.split_k)
+                    if na < 64 or 2 * groups > cus:
+                        assert p.split_k == 1, (bt, nn, na)
+                    elif na >= 128:  # half the units or more are at work, or the split is at its limits
+                        assert 2 * groups * p.split_k >= cus or p.split_k >= min(6, na // 16), (bt, nn, na, p.split_k)

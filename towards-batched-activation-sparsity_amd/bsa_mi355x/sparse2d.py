@@ -20,6 +20,7 @@ import torch
 from ._lib import Plan, check, load
 from .runtime import (BLOCK_K, MAX_NBLK, _cu_count, _dtype_code, _pad_k, _packed_entry, _require_cuda,
                       _sort_active_blocks_asc, _stream_handle, _workspace, ctypes_byref, resolve_plan)
+from .tuning import split_ways
 
 SORT_N_MAX = 512  # output-block list entries that the GEMM sorts itself (bsg_gemm_2d_sorted)
 INDEX_BLOCK_OUT_META_SIZE = 64  # output-block width of the 2-D path (KRN:19)
@@ -54,9 +55,11 @@ def plan_2d(bt: int, n_dim: int, nn: int, nblk: int, na: int, device: torch.devi
     full N (the tuned table), or the library's when that one is wider than 64 columns, and the
     split-K factor fills the chip without a partial second round: floor(CUs / work-groups),
     at most 4 for 32- and 64-row tiles (their partials are large) and 8 otherwise, measured on
-    down_proj B=16 and B=64 with 16-64 of 64 output blocks.  Up to 8 rows no split pays for its
-    hand-off: four list-splitting waves on 16 columns (K=N=4096, 32 x 20 blocks, 2 rows 6.3 us against
-    7.8 with split-K 3; K=11008, 60 x 32 blocks 8.7 / 9.8; N=22016, 16 x 300 blocks, 1 row 11.7 / 12.7).
+    down_proj B=16 and B=64 with 16-64 of 64 output blocks.  Up to 8 rows the tile is four
+    list-splitting waves on 16 columns (two for lists of fewer than 8 blocks: 3.1 us against 3.3 at 4
+    blocks), split further only where the blocks that this takes off each wave outweigh the hand-off
+    (tuning.split_ways): K=N=4096, 32 x 20 blocks, 2 rows 6.3 us unsplit, 7.8 with split-K 3; K=12288,
+    8 rows, 172 blocks x 3 output blocks 13.9 unsplit, 7.1 with split-K 8, x 32 15.7, 12.4 with 2.
     At 9-16 rows the 16-column tile widens while its tiles outnumber the compute units (K=4096
     N=11008, 32 x 86 blocks 10.2 / 11.8, 32 x 170 blocks 13.5 / 14.5; not past one 64-column tile per
     unit: N=22016, 30 x 300 blocks 21.8 / 20.3), and a split leaves each wave at
@@ -82,7 +85,7 @@ def plan_2d(bt: int, n_dim: int, nn: int, nblk: int, na: int, device: torch.devi
     if explicit and plan.split_k:
         return pl
     if not explicit and int(bt) <= 8:
-        return Plan(1, 16, 4, 4, 16, 1)
+        return Plan(split_ways(4 * nn, int(bt), int(na), _cu_count(device)), 16, 4 if na >= 8 else 2, 4, 16, 1)
     cols = pl.cols_per_wave
     if not explicit and pl.kind == 1 and pl.rows_per_group == 16 and nn <= _cu_count(device):
         while cols < BLOCK_N_OUT and max(1, nn) * (BLOCK_N_OUT // cols) > _cu_count(device):
