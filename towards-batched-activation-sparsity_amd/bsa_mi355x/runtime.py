@@ -212,15 +212,16 @@ def resolve_plan(bt: int, n: int, nblk: int, na: int, device: torch.device, plan
                  dense: bool = False, lookup_plan: bool = True, select: bool = False, sized: bool = True) -> Plan:
     """Resolve a (partial) plan for a problem.  With no plan (or an all-zero one) the tuned
     table (tuning.lookup; select=True: the entries timed as selection + GEMM first) is consulted
-    first, then (sized) the plan by size, tuning.sized_plan; remaining zero fields are filled by the library's heuristics; tile fields that name a
-    kernel that is not instantiated fall back to automatic (the split-K factor is kept)."""
+    first, then (sized) the plan by size, tuning.sized_plan; remaining zero fields are filled by the
+    library's heuristics; tile fields that name a kernel that is not instantiated fall back to
+    automatic (the split-K factor is kept)."""
     lib = load()
     if lookup_plan and (plan is None or not any(plan.as_tuple())):
         from . import tuning
 
         tuned = tuning.lookup(bt, n, nblk, na, dense=dense, select=select)
         if tuned is None and sized:
-            tuned = tuning.sized_plan(bt, n, na)
+            tuned = tuning.sized_plan(bt, n, na, _cu_count(device))
         if tuned is not None:
             plan = tuned
     req = plan.as_tuple() if plan is not None else (0, 0, 0, 0, 0, 0)

@@ -45,16 +45,17 @@ def rows_bucket(bt: int) -> int:
 
 def split_ways(tiles: int, rows: int, na: int, cus: int) -> int:
     """Work-groups that share each of `tiles` 16-column tiles of up to 16 rows, their four waves
-    splitting the list too.  By measurement (K=12288, 4 to 256 tiles, 16 to 192 blocks, 1 to 16 rows)
-    a block takes its wave 0.14 us and 0.014 more per row, and handing the partial sums on takes 1.7 us
-    and 2.6 ns per work-group: the count with the least of both, which leaves every wave at least 4
-    blocks and starts no more work-groups than there are compute units.  At each of those
-    points it is within 8% of the better of no split and two-wave groups split as widely as fits."""
-    best, best_us = 1, na / 4 * (0.14 + 0.014 * rows)
+    splitting the list too.  By measurement (K=12288, 4 to 256 tiles, 4 to 192 blocks, 1 to 16 rows)
+    a block takes its wave 0.14 us and 0.0115 more per row, and handing the partial sums on takes 1.5
+    us and 4 ns per work-group: the count with the least of both, which leaves every wave at least 4
+    blocks and starts no more work-groups than there are compute units.  At each of those points it
+    is within 11% of the better of no split and two-wave groups split as widely as fits."""
+    per_block = 0.14 + 0.0115 * rows
+    best, best_us = 1, na / 4 * per_block
     for s in range(2, 9):
         if tiles * s > cus or na < 16 * s:
             break
-        us = na / (4 * s) * (0.14 + 0.014 * rows) + 1.7 + 0.0026 * tiles * s
+        us = na / (4 * s) * per_block + 1.5 + 0.004 * tiles * s
         if us < best_us:
             best, best_us = s, us
     return best
@@ -82,7 +83,7 @@ def many_rows_plan(bt: int, n: int) -> Plan:
     return Plan(2, 32, 8, 4, 64, 4)
 
 
-def sized_plan(bt: int, n: int, na: int) -> Optional[Plan]:
+def sized_plan(bt: int, n: int, na: int, cus: int = _CUS) -> Plan:
     """Plan by size for a problem without a tuned one (a selection + GEMM, or a capture, of a shape
     the table does not hold): variable-width column groups of as many 16-column subtiles as one
     compute unit gets, which fill the chip at any width, where the library's heuristic rounds to 16
@@ -90,18 +91,24 @@ def sized_plan(bt: int, n: int, na: int) -> Optional[Plan]:
     kinds 7 and 5, to 64 kind 7.  Measured beside the heuristic, GEMM / selection + GEMM, us:
     N=2048 K=2048 16 blocks, 5 rows 3.6 against 5.5 / 7.4 against 11.9, 64 rows 4.9, 9.1 / 8.1, 12.0;
     N=13824 K=5120 32 blocks, 16 rows 13.1, 15.9 / 17.2, 21.3, 64 rows 16.0, 21.8 / 20.5, 26.5.
-    None (the heuristic) for long lists over few columns past 16 rows, where its split-K wins:
-    N=4096, 96 blocks, 24 / 48 rows 13.3 / 16.1 against 15.9 / 18.1, while N=3072, 89 blocks, takes
-    13.6 / 16.0 here against 14.2 / 18.8."""
+
+    With no more than one subtile per unit such a group walks the whole list for one subtile, so
+    long lists are split over the units instead: up to 16 rows as split_ways counts (N=1000, 192
+    blocks, 8 rows: 14.3 unsplit, 9.3 split), above on kind 2's 64 columns where the split takes
+    48 blocks (56 past 32 rows) or more off each work-group (N=1000, 24 / 64 rows: 128 blocks 14.8 / 18.4
+    unsplit, 10.0 / 13.4 split; 64 blocks 8.8 / 10.9, 8.0 / 10.6; N=4096, 64 blocks 10.6 / 12.5, 10.3 /
+    13.2)."""
     if bt > 64:
         return many_rows_plan(bt, n)
     tiles = -(-int(n) // 16)
-    s = -(-tiles // _CUS)
+    s = -(-tiles // cus)
     cols = 16 * (s if s <= 4 else 6)
-    if s == 1 and bt > 16 and na * tiles > 20000:
-        return None
     if bt <= 16:
-        return Plan(1, cols, 4, 4, 16, 6 if s == 1 else 5)
+        ways = split_ways(tiles, bt, na, cus)
+        return Plan(ways, 16, 4, 4, 16, 1) if ways > 1 else Plan(1, cols, 4, 4, 16, 6 if s == 1 else 5)
+    ways = min(8, cus // -(-int(n) // 64)) if s == 1 else 1
+    if ways > 1 and na * (ways - 1) >= (48 if bt <= 32 else 56) * ways:
+        return Plan(ways, 16, 4, 4, 32 if bt <= 32 else 64, 2)
     if bt <= 32:
         return Plan(1, 32, 4, 4, 16, 5) if s == 1 else Plan(1, cols, 4, 2, 32, 7) if s <= 4 else \
             Plan(1, 96, 4, 4, 32, 5)
