@@ -416,3 +416,31 @@ def test_sized_plans_split_long_lists_over_few_columns():
         # half the units hold N=2048 without a split where 256 split it two ways
         assert tuning.sized_plan(bt, 2048, 192, 256).split_k > 1
         assert tuning.sized_plan(min(bt, 16), 2048, 192, 128).split_k == 1
+
+
+def test_many_rows_plans_take_no_round_that_another_width_saves():
+    """Past 64 rows a kind-8 plan's column groups, counted as the launcher deals them, take no more
+    per compute unit over all rounds, rounds x (rows + columns), than any other kind-8 width; and the
+    sizes where a few groups past the unit count used to open a second round (timed, 31 blocks: N=16384,
+    256 rows 45.2 us with 96 columns, 36.7 with 64; N=4096, 192 rows 18.9 with 258 groups of 48 columns,
+    13.8 with 64; 320 rows 26.2 with 258 of kind 8, 16.9 with 64)."""
+    def cost(bt, n, nsub, cus):
+        yg, tiles = -(-bt // 128), -(-n // 16)
+        g = min(tiles, max(cus // yg, -(-tiles // nsub), 1))  # the launcher's groups per row group
+        return -(-g * yg // cus) * (128 + 16 * -(-tiles // g))
+
+    for cus in (256, 64):
+        for bt in (65, 72, 128, 129, 160, 192, 256, 320, 384, 512, 1024):
+            for n in (1000, 2048, 4096, 5120, 8192, 11008, 12288, 12304, 13827, 16384, 22016, 24592, 32000):
+                p = tuning.many_rows_plan(bt, n, cus=cus)
+                if p.kind == 8:
+                    best = min(cost(bt, n, nsub, cus) for nsub in (2, 3, 4, 6))
+                    assert cost(bt, n, p.cols_per_wave // 16, cus) <= best, (bt, n, cus, p.as_tuple())
+    for bt in (160, 256):
+        for n in (12304, 13827, 16384):
+            assert tuning.many_rows_plan(bt, n).as_tuple() == (1, 64, 8, 4, 128, 8)
+    assert tuning.many_rows_plan(192, 4096).as_tuple() == (1, 64, 4, 2, 64, 7)
+    assert tuning.many_rows_plan(320, 4096).as_tuple() == (1, 64, 8, 4, 128, 8)
+    assert tuning.many_rows_plan(256, 11008).as_tuple() == (1, 96, 8, 4, 128, 8)
+    # a lookup of a tabulated shape plans for the units it is given
+    assert tuning.lookup(256, 11008, 64, 31, cus=128).as_tuple() == tuning.many_rows_plan(256, 11008, 31, 128).as_tuple()

@@ -219,7 +219,7 @@ def resolve_plan(bt: int, n: int, nblk: int, na: int, device: torch.device, plan
     if lookup_plan and (plan is None or not any(plan.as_tuple())):
         from . import tuning
 
-        tuned = tuning.lookup(bt, n, nblk, na, dense=dense, select=select)
+        tuned = tuning.lookup(bt, n, nblk, na, dense=dense, select=select, cus=_cu_count(device))
         if tuned is None and sized:
             tuned = tuning.sized_plan(bt, n, na, _cu_count(device))
         if tuned is not None:
@@ -456,7 +456,7 @@ def _first_call_plan(bt: int, n_dim: int, nblk: int, na: int, mode: str, code: i
     None (table plan or library heuristics)."""
     from . import autotune, tuning
 
-    if tuning.lookup(bt, n_dim, nblk, na, dense=(mode == "dense")) is not None:
+    if tuning.lookup(bt, n_dim, nblk, na, dense=(mode == "dense"), cus=_cu_count(dev)) is not None:
         return None
     k = autotune.key(n_dim, nblk, bt, na, mode, code)
     pl = autotune.cached(k)

@@ -35,7 +35,7 @@ LLAMA2_7B_SHAPES = {"qkvo": (4096, 4096), "gate_up": (4096, 11008), "down": (110
 
 _TABLE: Optional[List[dict]] = None
 _INDEX: Dict[Tuple[int, int], List[dict]] = {}
-# lookup() answers per (bt, N, nblk, na, dense, select), cleared whenever a table is loaded
+# lookup() answers per (bt, N, nblk, na, dense, select, cus), cleared whenever a table is loaded
 _MEMO: Dict[tuple, Optional[tuple]] = {}
 
 
@@ -65,22 +65,38 @@ def split_ways(tiles: int, rows: int, na: int, cus: int) -> int:
 _CUS = 256
 
 
-def many_rows_plan(bt: int, n: int) -> Plan:
+def many_rows_plan(bt: int, n: int, na: int = 31, cus: int = _CUS) -> Plan:
     """Plan for more than 64 rows, by size.  What a compute unit takes in per K-block, (rows +
-    columns of its tile) x 128 bytes, bounds these launches.  Where 128-row groups leave at least
-    3 column subtiles to each compute unit, kind 8 takes them (N = 11008, 31 blocks: 256 rows 23.2
-    us against 43.6 with four 64-row groups, 128 rows 18.4 / 23.0, 72 rows 15.2 / 19.3; N = 22016,
-    128 rows 25.7 / 36.8).  Below that the tile is nearer square with 64 rows: kind 7 up to 3
-    subtiles (N = 4096, 128 rows: 9.8, kind 8 12.9), and past 3 the 128-column tile of kind 4 with
-    the list split in two (N = 4096, 256 rows: 31 blocks 14.5, 83 blocks 27.1; kind 8 14.7, 31.4)."""
+    columns of its tile) x 128 bytes, bounds these launches, so the tile is the one nearest a
+    square that a unit's share of the columns allows: s128 and s64 are the 16-column subtiles per
+    unit when the launch deals the columns over cus // row groups units (us, 31 blocks, K=4096).
+
+    From s128 = 4 on kind 8, 64 columns wide, or 96 where that takes less per unit over all its rounds,
+    rounds x (128 + columns): its ring leaves one work-group to a unit, so a few work-groups past cus
+    cost a whole round (N=11008, 256 rows, s128 = 6: 23.6 with 96 columns, 34.8 with 64; N=16384, 256
+    rows, s128 = 8, two rounds either way: 36.7 with 64, 45.2 with 96; N=4096, 320 rows: 16.9 with 64,
+    26.2 with 48).  At s128 = 3 kind 8 on 48 columns (N=11008, 72 rows: 16.0, kind 7 17.7; N=9216, 65
+    rows: 15.4 / 17.0), kind 7 where two full 64-row groups take less (s64 = 5: N=5120, 256 rows: 16.8 /
+    15.3).  Below, 64-row groups of kind 7 (N=4096, 128 rows: 9.6, kind 8 12.9; N=6912, 128 rows: 12.7,
+    kind 8 16.2).  Where the 64-row groups do not divide the units, kind 4 with a list of 48 blocks
+    or more split over them (64 blocks, N=4096, 160 rows: 20.0, kind 7 23.5; N=2048, 320 rows: 17.5 /
+    22.2; 20 blocks, N=3072, 192 rows: 11.2 / 10.0)."""
     tiles = -(-int(n) // 16)
-    s128 = -(-tiles * -(-int(bt) // 128) // _CUS)
-    if s128 >= 3:
-        return Plan(1, 48 if s128 == 3 else 64 if s128 == 4 else 96, 8, 4, 128, 8)
-    s64 = -(-tiles * -(-int(bt) // 64) // _CUS)
-    if s64 <= 3:
-        return Plan(1, 32 if s64 <= 2 else 48, 4, 2, 64, 7)
-    return Plan(2, 32, 8, 4, 64, 4)
+    yg128, yg64 = -(-int(bt) // 128), -(-int(bt) // 64)
+    s128 = -(-tiles // max(1, cus // yg128))
+    s64 = -(-tiles // max(1, cus // yg64))
+    if s128 >= 4:
+        def taken_in(nsub: int) -> int:
+            groups = max(cus // yg128, -(-tiles // nsub))
+            return -(-groups * yg128 // cus) * (128 + 16 * -(-tiles // groups))
+        return Plan(1, 96 if taken_in(6) < taken_in(4) else 64, 8, 4, 128, 8)
+    if s64 >= 3 and bt > 128 and cus % yg64:
+        ways = min(3, cus // (-(-int(n) // 128) * yg64))
+        if ways > 1 and na >= 48:
+            return Plan(ways, 32, 8, 4, 64, 4)
+    if s128 == 3 and (s64 != 5 or bt <= 112 * yg128):
+        return Plan(1, 48, 8, 4, 128, 8)
+    return Plan(1, 16 * max(2, s64), 4, 2, 64, 7) if s64 <= 4 else Plan(1, 96, 4, 3, 64, 7)
 
 
 def sized_plan(bt: int, n: int, na: int, cus: int = _CUS) -> Plan:
@@ -99,7 +115,7 @@ def sized_plan(bt: int, n: int, na: int, cus: int = _CUS) -> Plan:
     unsplit, 10.0 / 13.4 split; 64 blocks 8.8 / 10.9, 8.0 / 10.6; N=4096, 64 blocks 10.6 / 12.5, 10.3 /
     13.2)."""
     if bt > 64:
-        return many_rows_plan(bt, n)
+        return many_rows_plan(bt, n, na, cus)
     tiles = -(-int(n) // 16)
     s = -(-tiles // cus)
     cols = 16 * (s if s <= 4 else 6)
@@ -139,16 +155,17 @@ def load_table(path: str = TABLE_PATH) -> List[dict]:
     return entries
 
 
-def lookup(bt: int, n: int, nblk: int, na: int, dense: bool = False, select: bool = False) -> Optional[Plan]:
+def lookup(bt: int, n: int, nblk: int, na: int, dense: bool = False, select: bool = False,
+           cus: int = _CUS) -> Optional[Plan]:
     """Best tabulated plan for (bt, N, nblk, na): same N and block count, same 16/32/64-row
     bucket, nearest batch, then the dense entry (dense=True) or the nearest active-block count;
-    past 64 rows, the batches the table was tuned for, many_rows_plan.
+    past 64 rows, the batches the table was tuned for, many_rows_plan on `cus` compute units.
     select=True (a selection + GEMM, whose GEMM ranks the block scores itself) prefers the
     entries timed that way (refine_select) and falls back to the plain GEMM's.  None when the
     shape is not tabulated."""
     if _TABLE is None:
         load_table()
-    key = (int(bt), int(n), int(nblk), int(na), bool(dense), bool(select))
+    key = (int(bt), int(n), int(nblk), int(na), bool(dense), bool(select), int(cus))
     if key in _MEMO:
         hit = _MEMO[key]
         return None if hit is None else Plan(*hit)
@@ -157,12 +174,12 @@ def lookup(bt: int, n: int, nblk: int, na: int, dense: bool = False, select: boo
     return p
 
 
-def _lookup(bt: int, n: int, nblk: int, na: int, dense: bool, select: bool) -> Optional[Plan]:
+def _lookup(bt: int, n: int, nblk: int, na: int, dense: bool, select: bool, cus: int) -> Optional[Plan]:
     cands = _INDEX.get((n, nblk))
     if not cands:
         return None
     if bt > 64:
-        return many_rows_plan(bt, n)
+        return many_rows_plan(bt, n, na, cus)
     rb = rows_bucket(bt)
     same = [e for e in cands if rows_bucket(int(e["bt"])) == rb]
     if select and not dense:
