@@ -444,3 +444,20 @@ def test_many_rows_plans_take_no_round_that_another_width_saves():
     assert tuning.many_rows_plan(256, 11008).as_tuple() == (1, 96, 8, 4, 128, 8)
     # a lookup of a tabulated shape plans for the units it is given
     assert tuning.lookup(256, 11008, 64, 31, cus=128).as_tuple() == tuning.many_rows_plan(256, 11008, 31, 128).as_tuple()
+
+
+def test_selections_past_64_rows_rank_inside_the_gemm_where_the_tiles_tie():
+    """Kind 8 has no selection form, so a selection on it runs a rank launch of its own.  Where a unit
+    gets 3 subtiles of 128-row groups the 64-row tile takes no longer as a GEMM and ranks inside it
+    (N=11008, 128 rows: 21.6 us against 24.1), tabulated shape or not; plain GEMMs keep kind 8 there,
+    wider ones in both."""
+    for nblk in (64, 63):  # in the shipped table and not
+        for n in (11008, 12288):
+            for bt in (72, 96, 128):
+                tab = tuning.lookup(bt, n, nblk, 31, select=True)
+                sel = tab if tab is not None else tuning.sized_plan(bt, n, 31, select=True)
+                assert (tab is not None) == (nblk == 64) and sel.as_tuple() == (1, 96, 4, 3, 64, 7)
+                assert tuning.sized_plan(bt, n, 31).kind == 8
+                assert tuning.lookup(bt, n, 64, 31).kind == 8
+    assert tuning.lookup(96, 22016, 64, 31, select=True).kind == 8
+    assert tuning.sized_plan(256, 11008, 31, select=True).kind == 8

@@ -221,7 +221,7 @@ def resolve_plan(bt: int, n: int, nblk: int, na: int, device: torch.device, plan
 
         tuned = tuning.lookup(bt, n, nblk, na, dense=dense, select=select, cus=_cu_count(device))
         if tuned is None and sized:
-            tuned = tuning.sized_plan(bt, n, na, _cu_count(device))
+            tuned = tuning.sized_plan(bt, n, na, _cu_count(device), select)
         if tuned is not None:
             plan = tuned
     req = plan.as_tuple() if plan is not None else (0, 0, 0, 0, 0, 0)

@@ -65,7 +65,7 @@ def split_ways(tiles: int, rows: int, na: int, cus: int) -> int:
 _CUS = 256
 
 
-def many_rows_plan(bt: int, n: int, na: int = 31, cus: int = _CUS) -> Plan:
+def many_rows_plan(bt: int, n: int, na: int = 31, cus: int = _CUS, select: bool = False) -> Plan:
     """Plan for more than 64 rows, by size.  What a compute unit takes in per K-block, (rows +
     columns of its tile) x 128 bytes, bounds these launches, so the tile is the one nearest a
     square that a unit's share of the columns allows: s128 and s64 are the 16-column subtiles per
@@ -80,7 +80,10 @@ def many_rows_plan(bt: int, n: int, na: int = 31, cus: int = _CUS) -> Plan:
     15.3).  Below, 64-row groups of kind 7 (N=4096, 128 rows: 9.6, kind 8 12.9; N=6912, 128 rows: 12.7,
     kind 8 16.2).  Where the 64-row groups do not divide the units, kind 4 with a list of 48 blocks
     or more split over them (64 blocks, N=4096, 160 rows: 20.0, kind 7 23.5; N=2048, 320 rows: 17.5 /
-    22.2; 20 blocks, N=3072, 192 rows: 11.2 / 10.0)."""
+    22.2; 20 blocks, N=3072, 192 rows: 11.2 / 10.0).
+    A selection takes kind 7 at s128 = 3 too where its row groups divide the units: it ranks inside
+    the GEMM, where kind 8 needs a rank launch (N=11008, 72 / 96 / 128 rows: 21.2 / 21.3 / 21.6 against
+    21.1 / 22.1 / 24.1; N=12288 21.8 / 21.9 / 22.0, 21.3 / 22.2 / 24.2; N=2048, 640 rows 27.0 / 24.9)."""
     tiles = -(-int(n) // 16)
     yg128, yg64 = -(-int(bt) // 128), -(-int(bt) // 64)
     s128 = -(-tiles // max(1, cus // yg128))
@@ -94,12 +97,12 @@ def many_rows_plan(bt: int, n: int, na: int = 31, cus: int = _CUS) -> Plan:
         ways = min(3, cus // (-(-int(n) // 128) * yg64))
         if ways > 1 and na >= 48:
             return Plan(ways, 32, 8, 4, 64, 4)
-    if s128 == 3 and (s64 != 5 or bt <= 112 * yg128):
+    if s128 == 3 and (s64 != 5 or bt <= 112 * yg128) and not (select and cus % yg64 == 0):
         return Plan(1, 48, 8, 4, 128, 8)
     return Plan(1, 16 * max(2, s64), 4, 2, 64, 7) if s64 <= 4 else Plan(1, 96, 4, 3, 64, 7)
 
 
-def sized_plan(bt: int, n: int, na: int, cus: int = _CUS) -> Plan:
+def sized_plan(bt: int, n: int, na: int, cus: int = _CUS, select: bool = False) -> Plan:
     """Plan by size for a problem without a tuned one (a selection + GEMM, or a capture, of a shape
     the table does not hold): variable-width column groups of as many 16-column subtiles as one
     compute unit gets, which fill the chip at any width, where the library's heuristic rounds to 16
@@ -115,7 +118,7 @@ def sized_plan(bt: int, n: int, na: int, cus: int = _CUS) -> Plan:
     unsplit, 10.0 / 13.4 split; 64 blocks 8.8 / 10.9, 8.0 / 10.6; N=4096, 64 blocks 10.6 / 12.5, 10.3 /
     13.2)."""
     if bt > 64:
-        return many_rows_plan(bt, n, na, cus)
+        return many_rows_plan(bt, n, na, cus, select)
     tiles = -(-int(n) // 16)
     s = -(-tiles // cus)
     cols = 16 * (s if s <= 4 else 6)
@@ -179,7 +182,7 @@ def _lookup(bt: int, n: int, nblk: int, na: int, dense: bool, select: bool, cus:
     if not cands:
         return None
     if bt > 64:
-        return many_rows_plan(bt, n, na, cus)
+        return many_rows_plan(bt, n, na, cus, select and not dense)
     rb = rows_bucket(bt)
     same = [e for e in cands if rows_bucket(int(e["bt"])) == rb]
     if select and not dense:
