@@ -461,3 +461,34 @@ def test_selections_past_64_rows_rank_inside_the_gemm_where_the_tiles_tie():
                 assert tuning.lookup(bt, n, 64, 31).kind == 8
     assert tuning.lookup(96, 22016, 64, 31, select=True).kind == 8
     assert tuning.sized_plan(256, 11008, 31, select=True).kind == 8
+
+
+def test_lookup_honours_entries_tuned_past_64_rows(tmp_path):
+    """A table tuned for a batch past 64 rows answers such batches (nearest batch and block count, the
+    selection and dense entries as below), and no smaller one: a 64-row call never gets a kind-8 plan.
+    A shape tabulated for smaller batches only keeps the plan by size."""
+    e = {"N": 11008, "K": 4096, "dense": False, "us": 1.0}
+    path = tmp_path / "t.json"
+    path.write_text(json.dumps({"entries": [
+        dict(e, bt=128, na=31, plan=[1, 32, 8, 4, 128, 8]),
+        dict(e, bt=128, na=48, plan=[2, 32, 8, 4, 64, 4]),
+        dict(e, bt=128, na=31, select=True, plan=[1, 48, 4, 2, 64, 7]),
+        dict(e, bt=512, na=31, plan=[1, 64, 8, 4, 128, 8]),
+        dict(e, bt=96, N=4096, na=31, plan=[1, 32, 8, 4, 128, 8]),
+        dict(e, bt=64, N=2048, na=31, plan=[1, 32, 4, 2, 32, 7]),
+    ]}))
+    tuning.load_table(str(path))
+    try:
+        assert tuning.lookup(128, 11008, 64, 31).as_tuple() == (1, 32, 8, 4, 128, 8)
+        assert tuning.lookup(72, 11008, 64, 30).as_tuple() == (1, 32, 8, 4, 128, 8)
+        assert tuning.lookup(128, 11008, 64, 50).as_tuple() == (2, 32, 8, 4, 64, 4)
+        assert tuning.lookup(128, 11008, 64, 31, select=True).as_tuple() == (1, 48, 4, 2, 64, 7)
+        assert tuning.lookup(400, 11008, 64, 31).as_tuple() == (1, 64, 8, 4, 128, 8)
+        # no dense entry past 64 rows: by size
+        assert tuning.lookup(128, 11008, 64, 64, dense=True).as_tuple() == tuning.many_rows_plan(128, 11008, 64).as_tuple()
+        for bt in (1, 40, 64):
+            assert tuning.lookup(bt, 4096, 64, 31) is None
+        assert tuning.lookup(128, 2048, 64, 31).as_tuple() == tuning.many_rows_plan(128, 2048, 31).as_tuple()
+        assert tuning.lookup(48, 2048, 64, 31).as_tuple() == (1, 32, 4, 2, 32, 7)
+    finally:
+        tuning.load_table()

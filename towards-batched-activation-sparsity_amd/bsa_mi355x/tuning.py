@@ -160,9 +160,10 @@ def load_table(path: str = TABLE_PATH) -> List[dict]:
 
 def lookup(bt: int, n: int, nblk: int, na: int, dense: bool = False, select: bool = False,
            cus: int = _CUS) -> Optional[Plan]:
-    """Best tabulated plan for (bt, N, nblk, na): same N and block count, same 16/32/64-row
-    bucket, nearest batch, then the dense entry (dense=True) or the nearest active-block count;
-    past 64 rows, the batches the table was tuned for, many_rows_plan on `cus` compute units.
+    """Best tabulated plan for (bt, N, nblk, na): same N and block count, same bucket of batches (up
+    to 16, 32 and 64 rows, and more), nearest batch, then the dense entry (dense=True) or the nearest
+    active-block count.  Past 64 rows a shape without an entry of such a batch takes many_rows_plan
+    on `cus` compute units.
     select=True (a selection + GEMM, whose GEMM ranks the block scores itself) prefers the
     entries timed that way (refine_select) and falls back to the plain GEMM's.  None when the
     shape is not tabulated."""
@@ -182,9 +183,15 @@ def _lookup(bt: int, n: int, nblk: int, na: int, dense: bool, select: bool, cus:
     if not cands:
         return None
     if bt > 64:
-        return many_rows_plan(bt, n, na, cus, select and not dense)
+        p = _nearest([e for e in cands if int(e["bt"]) > 64], bt, na, dense, select)
+        return p if p is not None else many_rows_plan(bt, n, na, cus, select and not dense)
+    # entries past 64 rows may name kind 8, which takes no smaller batch
     rb = rows_bucket(bt)
-    same = [e for e in cands if rows_bucket(int(e["bt"])) == rb]
+    return _nearest([e for e in cands if int(e["bt"]) <= 64 and rows_bucket(int(e["bt"])) == rb], bt, na, dense, select)
+
+
+def _nearest(same: List[dict], bt: int, na: int, dense: bool, select: bool) -> Optional[Plan]:
+    """lookup's answer from the entries of one shape and batch bucket."""
     if select and not dense:
         sel = [e for e in same if e.get("select")]
         if sel:
@@ -202,7 +209,8 @@ def _lookup(bt: int, n: int, nblk: int, na: int, dense: bool, select: bool, cus:
     e = min(same, key=lambda e: (abs(int(e["na"]) - na), int(e["na"])))
     p = Plan(*[int(v) for v in e["plan"]])
     # a plan may split the batch into row groups only as it was tuned: groups of half the
-    # bucket's rows (16 in the 32-row bucket, 32 in the 64-row one); never smaller tiles
+    # bucket's rows (16 in the 32-row bucket, 32 in the 64-row one and past it); never smaller tiles
+    rb = rows_bucket(bt)
     if p.rows_per_group < min(bt, 64) and not (rb >= 32 and p.rows_per_group == rb // 2):
         return None
     return p
