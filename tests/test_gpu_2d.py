@@ -317,3 +317,29 @@ def test_2d_sorted_output_list_needs_memory_of_its_own(dev):
                            sort_active=True, n_sorted_out=buf[2:4])
     torch.cuda.synchronize()
     assert bool((y == SENTINEL).all()) and buf.tolist() == [9, 3, 5, 1, 0, 0]
+
+
+@pytest.mark.parametrize("plan", [None, (1, 16, 4, 4, 16, 1), (2, 16, 4, 4, 64, 2)])
+def test_2d_packed_entry_with_an_empty_k_list(dev, plan):
+    """No active K-block: the active output blocks are zero (not the dense product), whatever the
+    form of the empty list, sorted or not, in place and compact; the sorted ids are still written."""
+    bt, kdim, n = 5, 640, 1000
+    x, w_nk, _ = case(12, bt, kdim, n, 1, "normal")
+    packed, xt = bsa.pack_weight(to_dev(w_nk, dev)), to_dev(x, dev)
+    empty = torch.empty(0, dtype=torch.int32, device=dev)
+    some = torch.tensor([3, 4], dtype=torch.int32, device=dev)
+    nb = torch.tensor([15, 2, 7], dtype=torch.int32, device=dev)
+    p = bsa.Plan(*plan) if plan else None
+    on = torch.zeros(n, dtype=torch.bool, device=dev)
+    for b in nb.tolist():
+        on[64 * b:64 * b + 64] = True
+    for kb, kw in ((empty, {}), (some, {"num_active": 0})):
+        for sort in (False, True):
+            y = torch.full((bt, n), SENTINEL, dtype=torch.float16, device=dev)
+            c = torch.full((bt, 192), SENTINEL, dtype=torch.float16, device=dev)
+            for out, compact in ((y, False), (c, True)):
+                ids = torch.full((3,), -7, dtype=torch.int32, device=dev)
+                lists = {"sort_active": True, "n_sorted_out": ids} if sort else {}
+                s2d.gemm_2d_packed(xt, packed, n, kb, nb, out, compact=compact, plan=p, **kw, **lists)
+                assert not sort or ids.tolist() == [2, 7, 15]
+            assert not bool(y[:, on].any()) and bool((y[:, ~on] == SENTINEL).all()) and not bool(c.any())

@@ -110,9 +110,9 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
                    n_sorted_out: Optional[torch.Tensor] = None) -> Plan:
     """One 2-D block-sparse GEMM on packed weights (bsg_gemm_2d).
 
-    x2d [bt, K]; `active_blocks` int32 K-block list (None: every K-block) with optional host
-    length `num_active` and device count `num_active_dev`; `n_blocks` int32 list of active
-    64-column output blocks (ascending), host length `num_n`, optional device count
+    x2d [bt, K]; `active_blocks` int32 K-block list (None: every K-block; empty: a zero product)
+    with optional host length `num_active` and device count `num_active_dev`; `n_blocks` int32
+    list of active 64-column output blocks (ascending), host length `num_n`, optional device count
     `num_n_dev`.  sort_active: the GEMM sorts the K-block list ascending itself (at most
     MAX_NBLK // 2 entries); n_sorted_out (int32, at least num_n): n_blocks is in any order (at most
     SORT_N_MAX entries) and the GEMM takes its num_n lowest, writing them there ascending, while the
@@ -149,6 +149,9 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
             raise ValueError(f"{na} active K-blocks (list of {ab.numel()}, at most {MAX_NBLK})")
     else:
         ab, na = None, nblk
+    # the library takes a null list as every K-block; an empty list (no address of its own, and no
+    # entry that is read) passes the output-block list's address
+    ab_ptr = None if ab is None else ab.data_ptr() if na > 0 else nb.data_ptr()
     pl = plan_2d(bt, int(n_dim), nn, nblk, na, dev, plan, dense=active_blocks is None)
     ws_bytes = int(lib.bsg_gemm_workspace_bytes(bt, n_dim, ctypes_byref(pl)))
     ws_ptr = (_workspace(workspace_prefix, dev, ws_bytes, (bt, n_dim) + pl.as_tuple()).data_ptr()
@@ -157,13 +160,12 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
         if sort:
             check(lib.bsg_gemm_2d_sorted(
                 x2d.data_ptr(), x2d.stride(0), bt, x2d.shape[1], packed.data_ptr(), n_dim,
-                ab.data_ptr() if ab is not None and na > 0 else None, na if ab is not None else 0,
-                1 if sort_active else 0, nb.data_ptr(), int(nb.numel()), nn,
+                ab_ptr, na if ab is not None else 0, 1 if sort_active else 0, nb.data_ptr(), int(nb.numel()), nn,
                 n_sorted_out.data_ptr() if n_sorted_out is not None else None, 1 if compact else 0, y2d.data_ptr(),
                 y2d.stride(0), code, ws_ptr, ws_bytes, ctypes_byref(pl), _stream_handle(dev)))
             return pl
         rc = lib.bsg_gemm_2d(x2d.data_ptr(), x2d.stride(0), bt, x2d.shape[1], packed.data_ptr(), n_dim,
-                             ab.data_ptr() if ab is not None and na > 0 else None, na if ab is not None else 0,
+                             ab_ptr, na if ab is not None else 0,
                              num_active_dev.data_ptr() if num_active_dev is not None else None,
                              nb.data_ptr(), nn, num_n_dev.data_ptr() if num_n_dev is not None else None,
                              1 if compact else 0, y2d.data_ptr(), y2d.stride(0), code, ws_ptr, ws_bytes,
