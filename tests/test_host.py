@@ -492,3 +492,34 @@ def test_lookup_honours_entries_tuned_past_64_rows(tmp_path):
         assert tuning.lookup(48, 2048, 64, 31).as_tuple() == (1, 32, 4, 2, 32, 7)
     finally:
         tuning.load_table()
+
+
+def test_stale_prepared_entries_may_be_dropped_by_another_thread(monkeypatch):
+    """Two threads that find the same stale entry both drop it: the second goes on to the general
+    path (which refuses these CPU tensors) instead of failing on the missing key."""
+    import types
+
+    import torch
+
+    from bsa_mi355x import patch, runtime, select
+
+    x = torch.zeros(2, 1, 64, dtype=torch.float16)
+    w = torch.zeros(16, 64, dtype=torch.float16)
+    out = torch.zeros(2, 1, 16, dtype=torch.float16)
+    idx = torch.zeros(1, dtype=torch.int32)
+    stale = types.SimpleNamespace(wref=lambda: None, valid=lambda *a: False, ref=lambda: None)
+
+    class Raced(dict):  # every lookup finds a stale entry that is gone by the time it is dropped
+        def get(self, key, default=None):
+            return stale
+
+    for owner, name in ((runtime, "_PREPARED"), (select, "_PREPARED_SELECT"), (patch, "_PREPARED_LINEAR")):
+        monkeypatch.setattr(owner, name, Raced())
+    monkeypatch.setitem(runtime._WEIGHT_PREPACK_CACHE, "race", Raced())
+    not_on_gpu = "must live on"
+    with pytest.raises(ValueError, match=not_on_gpu):
+        bsa._prepacked_block_sparse_gemm_from_active_blocks(x, w, idx, out, cache_prefix="race")
+    with pytest.raises(ValueError, match=not_on_gpu):
+        bsa.select_sparse_gemm(x, w, out, 1, cache_prefix="race")
+    with pytest.raises(ValueError, match=not_on_gpu):
+        patch._fused_select_linear(x, w, out, 0.5, {"best_kern": "naive"}, "race", 64, None, 1.0, 0.1, None)

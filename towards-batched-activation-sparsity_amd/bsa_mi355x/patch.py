@@ -171,7 +171,7 @@ def _fused_select_linear(x3, weight, out, density: float, cfg: dict, cache_prefi
         if pc.valid(x3, weight, block_prior, block_score_scale):
             pc.call.launch(x3.data_ptr(), out.data_ptr(), torch._C._cuda_getCurrentRawStream(pc.dev_index))
             return
-        del _PREPARED_LINEAR[key]
+        _PREPARED_LINEAR.pop(key, None)  # another thread may have found the same stale entry
     if int(block_k) != INDEX_BLOCK_META_SIZE:
         raise ValueError(f"block_k must be {INDEX_BLOCK_META_SIZE}")
     n_out = out.shape[-1]

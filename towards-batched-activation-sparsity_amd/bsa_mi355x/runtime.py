@@ -125,7 +125,7 @@ def _packed_entry(weight: torch.Tensor, block_k: int, cache_prefix: str) -> _Pac
         if owner is not None and owner._version == entry.version:
             _WEIGHT_PREPACK_CACHE["hits"] += 1
             return entry
-        del cache[key]
+        cache.pop(key, None)
     _WEIGHT_PREPACK_CACHE["misses"] += 1
     packed = pack_weight(weight, "nk")
     entry = _PackEntry(packed, int(n_dim), int(m_dim), weakref.ref(weight), weight._version)
@@ -170,8 +170,8 @@ def release_prepacked_weights(cache_prefix: Optional[str] = None) -> None:
     for name, cache in list(_WEIGHT_PREPACK_CACHE.items()):
         if isinstance(cache, dict) and (cache_prefix is None or name == cache_prefix):
             cache.clear()
-    for key in [k for k in _PREPARED if cache_prefix is None or k[0] == cache_prefix]:
-        del _PREPARED[key]
+    for key in [k for k in list(_PREPARED) if cache_prefix is None or k[0] == cache_prefix]:
+        _PREPARED.pop(key, None)
     for hook in _FORGET_HOOKS:
         hook()
 
@@ -580,7 +580,7 @@ def _prepacked_block_sparse_gemm_from_active_blocks(
                 and torch._C._cuda_getDevice() == pc.dev_index):
             pc.launch(x, active_blocks, out)
             return
-        del _PREPARED[key]
+        _PREPARED.pop(key, None)  # another thread may have found the same stale entry
     n_dim = out.shape[-1]
     num_blocks = int(active_blocks.numel()) if active_blocks_limit is None else int(active_blocks_limit)
     num_blocks = min(num_blocks, int(active_blocks.numel()))

@@ -238,7 +238,7 @@ def select_sparse_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
                 if rc != _lib.BSG_OK:
                     check(rc)
                 return idx_out[:c.kk], count_out
-            del _PREPARED_SELECT[key]
+            _PREPARED_SELECT.pop(key, None)  # another thread may have found the same stale entry
     n_dim = out.shape[-1]
     x2d, y2d, bt, m_dim = _views(x, out, n_dim)
     _check_shapes(x2d, weight, y2d, n_dim, m_dim)
