@@ -523,3 +523,35 @@ def test_stale_prepared_entries_may_be_dropped_by_another_thread(monkeypatch):
         bsa.select_sparse_gemm(x, w, out, 1, cache_prefix="race")
     with pytest.raises(ValueError, match=not_on_gpu):
         patch._fused_select_linear(x, w, out, 0.5, {"best_kern": "naive"}, "race", 64, None, 1.0, 0.1, None)
+
+
+def test_prepared_calls_take_their_counts_by_value(monkeypatch):
+    """A block count given as a 0-d tensor or array is part of a prepared call's key by its value: an
+    array is not refused as unhashable, and a tensor changed in place is a different call."""
+    import numpy as np
+    import torch
+
+    from bsa_mi355x import runtime, select
+
+    seen = []
+
+    class Keys(dict):
+        def get(self, key, default=None):
+            seen.append(key)
+            return None
+
+    monkeypatch.setattr(select, "_PREPARED_SELECT", Keys())
+    monkeypatch.setattr(runtime, "_PREPARED", Keys())
+    x = torch.zeros(2, 1, 256, dtype=torch.float16)
+    w = torch.zeros(16, 256, dtype=torch.float16)
+    out = torch.zeros(2, 1, 16, dtype=torch.float16)
+    idx = torch.zeros(4, dtype=torch.int32)
+    count = torch.tensor(3)
+    for call in (lambda c: bsa.select_sparse_gemm(x, w, out, c),
+                 lambda c: bsa._prepacked_block_sparse_gemm_from_active_blocks(x, w, idx, out, active_blocks_limit=c)):
+        del seen[:]
+        for c, value in ((3, 3), (np.array(3), 3), (count, 3), (count, 2), (2, 2)):
+            count.fill_(value)
+            with pytest.raises(ValueError, match="must live on"):
+                call(c)
+        assert seen[0] == seen[1] == seen[2] and seen[3] == seen[4] and seen[0] != seen[3]

@@ -572,6 +572,8 @@ def _prepacked_block_sparse_gemm_from_active_blocks(
     launch: the packed weight, plan and workspace resolved by its first call, with only the
     weight's identity and version, the alignment and contiguity of x, out and the list, and the
     current device re-checked before the one library call."""
+    if active_blocks_limit is not None:
+        active_blocks_limit = int(active_blocks_limit)  # by value, also when given as a tensor or array
     key = _prepared_key(x, weight, active_blocks, out, cache_prefix, sort_active_blocks, active_blocks_limit)
     pc = _PREPARED.get(key)
     if pc is not None:

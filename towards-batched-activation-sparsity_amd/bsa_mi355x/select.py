@@ -220,6 +220,7 @@ def select_sparse_gemm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
     returns the (device) selected list and count.  A repeated exact-L1 call site without a plan
     takes a prepared launch (one library call: 17.2 -> 6.7 us a call at q/k/v/o B=1)."""
     key = None
+    k = int(k)  # a count given as a tensor or array is taken by value, as by a first call
     if score == "l1" and not rule and plan is None:
         key = (cache_prefix, id(weight), x.shape, x.stride(), x.dtype, x.get_device(), out.shape, out.dtype,
                out.get_device(), k)
