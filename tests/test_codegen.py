@@ -11,6 +11,8 @@ that no result test can pin reliably (CPU only: hipcc cross-compiles the device 
 - Kind 8 waits for a ring stage by the count of loads every wave issues per slot, so between two
   barriers of its pipeline each wave must issue exactly that many, whatever its lanes' bounds (a
   branch around a load would change the count), and must not wait for all of them.
+- The list sort (an LDS bitmap, set by LDS atomics) is in the sorting forms of a tile only: inlined
+  into the forms that take an ascending list it cost every launch of theirs 1-2%, the 2-D ones 2-9%.
 """
 from __future__ import annotations
 
@@ -114,3 +116,15 @@ def test_rows_kernel_issues_whole_stages_between_barriers(tmp_path):
         assert len(labels) <= 1 and not any("s_cbranch_exec" in x for x in pipe), name
         checked += 1
     assert checked == 8
+
+
+def test_only_the_sorting_forms_carry_the_sort(tmp_path):
+    asm = _device_asm("tiles_k4.hip", tmp_path)
+    seen = {}
+    for name, body in _functions(asm, "_ZN12_GLOBAL__N_118bsg_gemm_xl_kernel"):
+        form = int(re.findall(r"Li(\d+)E", name)[-1])  # none, top-k, budget, sort
+        n2d = "Lb1E" in name
+        seen.setdefault((form, n2d), 0)
+        seen[form, n2d] += 1
+        assert any("ds_or" in line for line in body) == (form == 3), name
+    assert set(seen) == {(0, False), (0, True), (1, False), (2, False), (3, False), (3, True)}

@@ -61,15 +61,18 @@ typedef void (*GemmFn)(GemmParams);
 
 enum { KIND_KSPLIT = 1, KIND_XLDS = 2, KIND_FMA = 3, KIND_XLDS_KH = 4, KIND_VT = 5, KIND_VT1 = 6, KIND_VT1X = 7, KIND_ROWS = 8 };
 
-// 1-D and, for tiles of at most 64 columns per work-group, 2-D (active output blocks) entries.
-// f16_sel, bf16_sel: the 1-D form compiled with the in-GEMM top-k (MODE_TOPK; in fp16 on 16-row
-// tiles also the self-scored MODE_TOPK_SELF), for the MFMA kinds (null for kinds 3 and 8); f16_bud,
-// bf16_bud: with the top-k under an energy budget (MODE_TOPK_BUDGET).  Every form leaves out what it
-// does not run: the top-k carried in every kernel cost every plain launch 0.1-0.2 us, and the
-// budget carried in the top-k kernels drained the loops of some (decode step 579 -> 658 us).
+// The compiled forms of a tile: 1-D, and for tiles of at most 64 columns per work-group 2-D (active
+// output blocks), each also as the form that sorts its lists (_sort); f16_sel, bf16_sel: the 1-D form
+// with the in-GEMM top-k (MODE_TOPK; in fp16 on 16-row tiles also the self-scored MODE_TOPK_SELF), for
+// the MFMA kinds (null for kinds 3 and 8); f16_bud, bf16_bud: with the top-k under an energy budget
+// (MODE_TOPK_BUDGET).  Every tile has every form that its kind can run, since a caller may name any
+// tile for any call.  Every form leaves out what it does not run: the top-k carried in every kernel
+// cost every plain launch 0.1-0.2 us, and the budget carried in the top-k kernels drained the loops
+// of some (decode step 579 -> 658 us).
 struct KernelEntry {
   int kind, rows, nsub, wpg, depth;
-  GemmFn f16, bf16, f16_2d, bf16_2d, f16_sel, bf16_sel, f16_bud, bf16_bud;
+  GemmFn f16, bf16, f16_sort, bf16_sort, f16_2d, bf16_2d, f16_2d_sort, bf16_2d_sort;
+  GemmFn f16_sel, bf16_sel, f16_bud, bf16_bud;
 };
 
 // A translation unit's slice of the instantiated tile set.
@@ -147,8 +150,10 @@ enum { MODE_LIST = 0, MODE_BITMAP = 1, MODE_DENSE = 2, MODE_TOPK = 3, MODE_TOPK_
 // A GEMM ranks block scores itself (MODE_TOPK) up to this many blocks: keys and ranks fit its
 // block-list buffer, and a one-wave work-group flags at most 8 per thread.
 #define BSG_TOPK_MAX_NBLK 512
-// What selection code a kernel form carries (KernelEntry).
-enum { SEL_NONE = 0, SEL_TOPK = 1, SEL_BUDGET = 2 };
+// What selection or sorting code a kernel form carries (KernelEntry); SEL_ANY_LIST: the sort beside
+// every other list source.
+enum { SEL_NONE = 0, SEL_TOPK = 1, SEL_BUDGET = 2, SEL_SORT = 3, SEL_ANY_LIST = 4 };
+constexpr bool sel_sorts(int sel) { return sel == SEL_SORT || sel == SEL_ANY_LIST; }
 #define BSG_SELF_MAX_ROWS 8
 
 // The 2-D kernels sort an output-block list of up to this many entries themselves.
@@ -580,7 +585,7 @@ __device__ __forceinline__ int nth_output_block(const GemmParams& p, int bi) {
 // the tile has no block (past the device-side count): the whole work-group then returns
 // before any barrier.  A block id outside [0, ceil(N/64)) reads past the packed columns (zero
 // weights) and writes nothing.
-template <bool N2D, int NT>
+template <bool N2D, int NT, int SEL>
 __device__ __forceinline__ bool tile_columns(const GemmParams& p, int tile, int gc, int* n0, int* n0y) {
   if constexpr (!N2D) {
     *n0 = *n0y = tile * gc;
@@ -595,7 +600,12 @@ __device__ __forceinline__ bool tile_columns(const GemmParams& p, int tile, int 
     }
     if (bi >= nn) return false;
     const int off = (tile - bi * per) * gc;
-    const int nb = __builtin_amdgcn_readfirstlane(p.idx_out != nullptr ? nth_output_block<NT>(p, bi) : p.nidx[bi]);
+    int id;
+    if constexpr (sel_sorts(SEL))
+      id = p.idx_out != nullptr ? nth_output_block<NT>(p, bi) : p.nidx[bi];
+    else
+      id = p.nidx[bi];
+    const int nb = __builtin_amdgcn_readfirstlane(id);
     const bool ok = nb >= 0 && nb < (p.N + 63) / 64;
     *n0 = ok ? nb * 64 + off : p.npad;
     *n0y = p.ncompact ? bi * 64 + off : (ok ? *n0 : p.ny);
@@ -736,17 +746,22 @@ __device__ __forceinline__ void sort_block_list(const int32_t* ids, int na, int 
 }
 
 // This thread's entry of a list the kernel is to sort, requested at kernel entry (a list whose
-// length is on the device is read once the length is known).
+// length is on the device is read once the length is known); the sorting forms only.
+template <int SEL>
 __device__ __forceinline__ int list_entry_of_thread(const GemmParams& p) {
+  if constexpr (!sel_sorts(SEL)) return 0;
   return p.sort_list && p.na_dev == nullptr && (int)threadIdx.x < p.na ? p.idx[threadIdx.x] : 0;
 }
 
 // Stage this call's active-block list in LDS (list copy, bitmap compaction, top-k of block
 // scores or identity) and return its length.  Ends with a barrier.  s_ids is 16-byte aligned
 // and holds BSG_MAX_NBLK ids; the top-k stages its keys in the first half and its ranks in the
-// second (up to 512 blocks).  SEL: only the in-GEMM top-k is compiled in (SELF_SCORE: also its
-// self-scored form), in the selection forms of KernelEntry, which are launched in those modes only;
-// without the list, bitmap and dense branches beside it the selection + GEMM calls take 2-4% less.
+// second (up to 512 blocks).  SEL: the code of a KernelEntry form, which is launched in its modes
+// only.  The selection forms carry the in-GEMM top-k (SELF_SCORE: also its self-scored form) and
+// nothing else: without the list, bitmap and dense branches beside it the selection + GEMM calls
+// take 2-4% less.  The plain forms carry no sort: with one inlined, launches on ascending lists took
+// longer (q/k/v/o 13 blocks, 2 rows 3.71 us against 3.62; down 83 blocks, 64 rows 15.63 / 15.25; 2-D
+// q/k/v/o 64 rows 9.81 / 9.10), and the sorting forms no bitmap.
 template <int NT, int SEL = SEL_NONE, bool SELF_SCORE = false>
 __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids, int first) {
   const int tid = threadIdx.x;
@@ -771,13 +786,16 @@ __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids,
     if (p.na_dev != nullptr) {
       const int d = *p.na_dev;
       na = d < 0 ? 0 : (d < na ? d : na);
-      if (p.sort_list && tid < na) first = p.idx[tid];
+      if (sel_sorts(SEL) && p.sort_list && tid < na) first = p.idx[tid];
     }
-    if (p.sort_list)
-      sort_block_list<NT>(p.idx, __builtin_amdgcn_readfirstlane(na), p.nblk, first, s_ids);
-    else
+    bool sorted = false;
+    if constexpr (sel_sorts(SEL)) {
+      sorted = p.sort_list != 0;
+      if (sorted) sort_block_list<NT>(p.idx, __builtin_amdgcn_readfirstlane(na), p.nblk, first, s_ids);
+    }
+    if (!sorted)
       for (int i = tid; i < na; i += NT) s_ids[i] = p.idx[i];
-  } else if (p.mode == MODE_BITMAP) {
+  } else if (SEL != SEL_SORT && p.mode == MODE_BITMAP) {
     // Every wave ballots the flags of each 64-block group and keeps the running count, so a
     // block's position needs no scan over the work-group; wave g % W writes group g.  The flags of
     // U groups are requested together.
@@ -804,7 +822,7 @@ __device__ __forceinline__ int stage_block_list(const GemmParams& p, int* s_ids,
   }
   na = __builtin_amdgcn_readfirstlane(na);
   __syncthreads();
-  if (SEL != SEL_NONE && p.idx_out != nullptr && blockIdx.x == 0 && blockIdx.y == 0) {
+  if ((SEL == SEL_TOPK || SEL == SEL_BUDGET) && p.idx_out != nullptr && blockIdx.x == 0 && blockIdx.y == 0) {
     for (int i = tid; i < na; i += NT) p.idx_out[i] = s_ids[i];
     if (tid == 0) *p.na_out = na;
   }
@@ -933,9 +951,9 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_kernel(GemmParams p) {
   int tile, sk;
   tile_of_group(p.split_k, &tile, &sk);
   const int S = p.split_k;
-  const int first = list_entry_of_thread(p);
+  const int first = list_entry_of_thread<SEL>(p);
   int n0, n0y;
-  if (!tile_columns<N2D, NT>(p, tile, 16 * NSUB, &n0, &n0y)) return;
+  if (!tile_columns<N2D, NT, SEL>(p, tile, 16 * NSUB, &n0, &n0y)) return;
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
@@ -1102,9 +1120,9 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
   int tile, sk;
   tile_of_group(p.split_k, &tile, &sk);
   const int S = p.split_k;
-  const int first = list_entry_of_thread(p);
+  const int first = list_entry_of_thread<SEL>(p);
   int n0, n0y;
-  if (!tile_columns<N2D, NT>(p, tile, 16 * CS, &n0, &n0y)) return;
+  if (!tile_columns<N2D, NT, SEL>(p, tile, 16 * CS, &n0, &n0y)) return;
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
@@ -1254,7 +1272,7 @@ __global__ __launch_bounds__(64 * WC * WK) void bsg_gemm_xl_kernel(GemmParams p)
 // each of its later reads is a broadcast and the loop streams weights only.  A wave reads only
 // what it wrote, and one wave's LDS accesses complete in order, so the staging needs no
 // barrier.  The waves are reduced through LDS in wave order.
-template <typename T, int BT, int NSUB, int WPG, int DEPTH, bool N2D>
+template <typename T, int BT, int NSUB, int WPG, int DEPTH, bool N2D, int SEL = SEL_NONE>
 __global__ __launch_bounds__(64 * WPG) void bsg_gemm_fma_kernel(GemmParams p) {
   constexpr int NT = 64 * WPG;
   constexpr int XI = BSG_FMA_X_LOADS;  // staging loads per wave (host guarantees enough)
@@ -1265,14 +1283,14 @@ __global__ __launch_bounds__(64 * WPG) void bsg_gemm_fma_kernel(GemmParams p) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = blockIdx.x;
-  const int first = list_entry_of_thread(p);
+  const int first = list_entry_of_thread<SEL>(p);
   int n0, n0y;
-  if (!tile_columns<N2D, NT>(p, tile, 16 * NSUB, &n0, &n0y)) return;
+  if (!tile_columns<N2D, NT, SEL>(p, tile, 16 * NSUB, &n0, &n0y)) return;
   const int y0 = blockIdx.y * BT;
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT>(p, s_ids, first);
+  const int na = stage_block_list<NT, SEL>(p, s_ids, first);
   BSG_TL(1);
   const int pbeg = (int)(((int64_t)na * w) / WPG);
   const int pend = (int)(((int64_t)na * (w + 1)) / WPG);
@@ -1476,7 +1494,7 @@ __global__ __launch_bounds__(64 * KH * WB) void bsg_gemm_vt_kernel(GemmParams p)
   tile_of_group(1, &tile, &sk);
   int st, nv;
   vt_columns(tile, p.n_tiles, p.npad >> 4, &st, &nv);
-  const int first = list_entry_of_thread(p);
+  const int first = list_entry_of_thread<SEL>(p);
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
@@ -1612,7 +1630,7 @@ __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   tile_of_group(1, &tile, &sk);
   int st, nv;
   vt_columns(tile, p.n_tiles, p.npad >> 4, &st, &nv);
-  const int first = list_entry_of_thread(p);
+  const int first = list_entry_of_thread<SEL>(p);
   const int y0 = blockIdx.y * (16 * BTT);
   BSG_TL_DECL
   BSG_TL(0);
@@ -1753,27 +1771,27 @@ __global__ __launch_bounds__(64 * WB) void bsg_gemm_vtx_kernel(GemmParams p) {
   BSG_TL_END(p, true);
 }
 
-// The 2-D instantiation of a tile, or null when its work-group covers more than one 64-column
-// output block (the discarded branch is never instantiated).
-template <int KIND, typename T, int B, int S, int W, int D>
+// The 2-D instantiation of a tile (SEL_NONE or SEL_SORT), or null when its work-group covers more
+// than one 64-column output block (the discarded branch is never instantiated).
+template <int KIND, typename T, int SEL, int B, int S, int W, int D>
 constexpr GemmFn kernel_2d() {
   constexpr int gc = KIND == KIND_XLDS ? 16 * S * W : (KIND == KIND_XLDS_KH ? 16 * S * (W / 2) : 16 * S);
   if constexpr (gc > 64) {
     return nullptr;
   } else if constexpr (KIND == KIND_KSPLIT) {
-    return bsg_gemm_kernel<T, B, S, W, D, true>;
+    return bsg_gemm_kernel<T, B, S, W, D, true, SEL>;
   } else if constexpr (KIND == KIND_XLDS) {
-    return bsg_gemm_xl_kernel<T, B, S, W, 1, D, true>;
+    return bsg_gemm_xl_kernel<T, B, S, W, 1, D, true, SEL>;
   } else if constexpr (KIND == KIND_XLDS_KH) {
-    return bsg_gemm_xl_kernel<T, B, S, W / 2, 2, D, true>;
+    return bsg_gemm_xl_kernel<T, B, S, W / 2, 2, D, true, SEL>;
   } else {
-    return bsg_gemm_fma_kernel<T, B, S, W, D, true>;
+    return bsg_gemm_fma_kernel<T, B, S, W, D, true, SEL>;
   }
 }
 
-// A selection form (1-D, in-GEMM top-k, SEL_TOPK or SEL_BUDGET) of a tile of the MFMA kinds.
+// The 1-D form of a tile that carries SEL's code.
 template <int KIND, typename T, int SEL, int B, int S, int W, int D>
-constexpr GemmFn kernel_sel() {
+constexpr GemmFn kernel_1d() {
   if constexpr (KIND == KIND_KSPLIT) {
     return bsg_gemm_kernel<T, B, S, W, D, false, SEL>;
   } else if constexpr (KIND == KIND_XLDS) {
@@ -1784,37 +1802,34 @@ constexpr GemmFn kernel_sel() {
     return bsg_gemm_vt_kernel<T, B, S, W / 2, D, 2, SEL>;
   } else if constexpr (KIND == KIND_VT1) {
     return bsg_gemm_vt_kernel<T, B, S, W, D, 1, SEL>;
-  } else {
+  } else if constexpr (KIND == KIND_VT1X) {
     return bsg_gemm_vtx_kernel<T, B, S, W, D, SEL>;
+  } else {
+    return bsg_gemm_fma_kernel<T, B, S, W, D, false, SEL>;
   }
 }
 
-#define BSG_SEL_FORMS(KIND, B, S, W, D)                                                          \
-  kernel_sel<KIND, _Float16, SEL_TOPK, B, S, W, D>(), kernel_sel<KIND, __bf16, SEL_TOPK, B, S, W, D>(), \
-      kernel_sel<KIND, _Float16, SEL_BUDGET, B, S, W, D>(), kernel_sel<KIND, __bf16, SEL_BUDGET, B, S, W, D>()
-#define BSG_K(B, S, W, D)                                                                                          \
-  {KIND_KSPLIT, 16 * B, S, W, D, bsg_gemm_kernel<_Float16, B, S, W, D, false>, bsg_gemm_kernel<__bf16, B, S, W, D, false>, \
-   kernel_2d<KIND_KSPLIT, _Float16, B, S, W, D>(), kernel_2d<KIND_KSPLIT, __bf16, B, S, W, D>(),                   \
-   BSG_SEL_FORMS(KIND_KSPLIT, B, S, W, D)}
-#define BSG_X(B, S, W, D)                                                                     \
-  {KIND_XLDS, 16 * B, S, W, D, bsg_gemm_xl_kernel<_Float16, B, S, W, 1, D, false>,           \
-   bsg_gemm_xl_kernel<__bf16, B, S, W, 1, D, false>, kernel_2d<KIND_XLDS, _Float16, B, S, W, D>(), \
-   kernel_2d<KIND_XLDS, __bf16, B, S, W, D>(), BSG_SEL_FORMS(KIND_XLDS, B, S, W, D)}
-#define BSG_Y(B, S, W, D)                                                                        \
-  {KIND_XLDS_KH, 16 * B, S, W, D, bsg_gemm_xl_kernel<_Float16, B, S, W / 2, 2, D, false>,        \
-   bsg_gemm_xl_kernel<__bf16, B, S, W / 2, 2, D, false>, kernel_2d<KIND_XLDS_KH, _Float16, B, S, W, D>(), \
-   kernel_2d<KIND_XLDS_KH, __bf16, B, S, W, D>(), BSG_SEL_FORMS(KIND_XLDS_KH, B, S, W, D)}
-#define BSG_V(B, S, W, D)                                                                               \
-  {KIND_VT, 16 * B, S, W, D, bsg_gemm_vt_kernel<_Float16, B, S, W / 2, D>, bsg_gemm_vt_kernel<__bf16, B, S, W / 2, D>, \
-   nullptr, nullptr, BSG_SEL_FORMS(KIND_VT, B, S, W, D)}
-#define BSG_V1(B, S, W, D)                                                                                \
-  {KIND_VT1, 16 * B, S, W, D, bsg_gemm_vt_kernel<_Float16, B, S, W, D, 1>, bsg_gemm_vt_kernel<__bf16, B, S, W, D, 1>, \
-   nullptr, nullptr, BSG_SEL_FORMS(KIND_VT1, B, S, W, D)}
-#define BSG_V1X(B, S, W, D)                                                                                    \
-  {KIND_VT1X, 16 * B, S, W, D, bsg_gemm_vtx_kernel<_Float16, B, S, W, D>, bsg_gemm_vtx_kernel<__bf16, B, S, W, D>, \
-   nullptr, nullptr, BSG_SEL_FORMS(KIND_VT1X, B, S, W, D)}
-#define BSG_F(R, S, W, D)                                                                                 \
-  {KIND_FMA, R, S, W, D, bsg_gemm_fma_kernel<_Float16, R, S, W, D, false>, bsg_gemm_fma_kernel<__bf16, R, S, W, D, false>, \
-   kernel_2d<KIND_FMA, _Float16, R, S, W, D>(), kernel_2d<KIND_FMA, __bf16, R, S, W, D>(), nullptr, nullptr, nullptr, nullptr}
+// A form's fp16 and bf16 kernels, and the initializers of a tile's forms in KernelEntry's order.
+#define BSG_1D(KIND, SEL, ...) kernel_1d<KIND, _Float16, SEL, __VA_ARGS__>(), kernel_1d<KIND, __bf16, SEL, __VA_ARGS__>()
+#define BSG_2D(KIND, SEL, ...) kernel_2d<KIND, _Float16, SEL, __VA_ARGS__>(), kernel_2d<KIND, __bf16, SEL, __VA_ARGS__>()
+#define BSG_LIST_FORMS(KIND, ...) BSG_1D(KIND, SEL_NONE, __VA_ARGS__), BSG_1D(KIND, SEL_SORT, __VA_ARGS__)
+#define BSG_2D_FORMS(KIND, ...) BSG_2D(KIND, SEL_NONE, __VA_ARGS__), BSG_2D(KIND, SEL_SORT, __VA_ARGS__)
+#define BSG_NO_2D_FORMS nullptr, nullptr, nullptr, nullptr
+#define BSG_SEL_FORMS(KIND, ...) BSG_1D(KIND, SEL_TOPK, __VA_ARGS__), BSG_1D(KIND, SEL_BUDGET, __VA_ARGS__)
+#define BSG_NO_SEL_FORMS nullptr, nullptr, nullptr, nullptr
+
+#define BSG_TILE(KIND, R, B, S, W, D, FORMS_2D, SEL_FORMS) \
+  {KIND, R, S, W, D, BSG_LIST_FORMS(KIND, B, S, W, D), FORMS_2D, SEL_FORMS}
+#define BSG_K(B, S, W, D) \
+  BSG_TILE(KIND_KSPLIT, 16 * B, B, S, W, D, BSG_2D_FORMS(KIND_KSPLIT, B, S, W, D), BSG_SEL_FORMS(KIND_KSPLIT, B, S, W, D))
+#define BSG_X(B, S, W, D) \
+  BSG_TILE(KIND_XLDS, 16 * B, B, S, W, D, BSG_2D_FORMS(KIND_XLDS, B, S, W, D), BSG_SEL_FORMS(KIND_XLDS, B, S, W, D))
+#define BSG_Y(B, S, W, D)                                                           \
+  BSG_TILE(KIND_XLDS_KH, 16 * B, B, S, W, D, BSG_2D_FORMS(KIND_XLDS_KH, B, S, W, D), \
+           BSG_SEL_FORMS(KIND_XLDS_KH, B, S, W, D))
+#define BSG_V(B, S, W, D) BSG_TILE(KIND_VT, 16 * B, B, S, W, D, BSG_NO_2D_FORMS, BSG_SEL_FORMS(KIND_VT, B, S, W, D))
+#define BSG_V1(B, S, W, D) BSG_TILE(KIND_VT1, 16 * B, B, S, W, D, BSG_NO_2D_FORMS, BSG_SEL_FORMS(KIND_VT1, B, S, W, D))
+#define BSG_V1X(B, S, W, D) BSG_TILE(KIND_VT1X, 16 * B, B, S, W, D, BSG_NO_2D_FORMS, BSG_SEL_FORMS(KIND_VT1X, B, S, W, D))
+#define BSG_F(R, S, W, D) BSG_TILE(KIND_FMA, R, R, S, W, D, BSG_2D_FORMS(KIND_FMA, R, S, W, D), BSG_NO_SEL_FORMS)
 
 }  // namespace

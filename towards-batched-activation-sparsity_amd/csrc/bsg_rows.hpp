@@ -24,7 +24,7 @@ __device__ __forceinline__ u32x4* ring_stage() {
 // arrival is one wait by count and one barrier.  The waves are row halves x channel halves: each
 // reads its rows' activation pieces and every weight piece of its channel half, and the channel
 // halves meet in LDS at the end, in the ring's storage.
-template <typename T, int BTT, int NSUB, int RW, int DEPTH>
+template <typename T, int BTT, int NSUB, int RW, int DEPTH, int SEL>
 __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
   constexpr int NW = 2 * RW;
   constexpr int NT = 64 * NW;
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
   BSG_TL_DECL
   BSG_TL(0);
 
-  const int na = stage_block_list<NT>(p, s_ids, list_entry_of_thread(p));
+  const int na = stage_block_list<NT, SEL>(p, s_ids, list_entry_of_thread<SEL>(p));
   BSG_TL(1);
 
   const int blk_bytes = p.npad * 128;
@@ -194,8 +194,11 @@ __global__ __launch_bounds__(128 * RW) void bsg_gemm_rows_kernel(GemmParams p) {
   BSG_TL_END(p, true);
 }
 
-#define BSG_R(B, S, RW, D)                                                                                       \
-  {KIND_ROWS, 16 * B, S, 2 * RW, D, bsg_gemm_rows_kernel<_Float16, B, S, RW, D>, bsg_gemm_rows_kernel<__bf16, B, S, RW, D>, \
-   nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}
+// One form for every list source: beside these launches (15 us and more) the sort's code does not show.
+#define BSG_R_FORM(...) \
+  bsg_gemm_rows_kernel<_Float16, __VA_ARGS__, SEL_ANY_LIST>, bsg_gemm_rows_kernel<__bf16, __VA_ARGS__, SEL_ANY_LIST>
+#define BSG_R(B, S, RW, D)                                                                       \
+  {KIND_ROWS, 16 * B, S, 2 * RW, D, BSG_R_FORM(B, S, RW, D), BSG_R_FORM(B, S, RW, D), BSG_NO_2D_FORMS, \
+   BSG_NO_SEL_FORMS}
 
 }  // namespace

@@ -843,10 +843,14 @@ int launch_gemm(int mode, const void* x, int64_t ldx, int64_t bt, int64_t K, con
   }
   dim3 block((unsigned)(64 * pl.waves_per_group), 1, 1);
   const bool topk = mode == MODE_TOPK || mode == MODE_TOPK_SELF || mode == MODE_TOPK_BUDGET;
-  GemmFn fn = mode == MODE_TOPK_BUDGET ? (dtype == BSG_F16 ? ke->f16_bud : ke->bf16_bud)
-              : topk ? (dtype == BSG_F16 ? ke->f16_sel : ke->bf16_sel)
-              : ex.nidx != nullptr ? (dtype == BSG_F16 ? ke->f16_2d : ke->bf16_2d)
-                                   : (dtype == BSG_F16 ? ke->f16 : ke->bf16);
+  const bool sorts = p.sort_list || ex.nidx_out != nullptr;
+  auto form = [&](GemmFn f16, GemmFn bf16) { return dtype == BSG_F16 ? f16 : bf16; };
+  GemmFn fn = mode == MODE_TOPK_BUDGET ? form(ke->f16_bud, ke->bf16_bud)
+              : topk                   ? form(ke->f16_sel, ke->bf16_sel)
+              : ex.nidx != nullptr && sorts ? form(ke->f16_2d_sort, ke->bf16_2d_sort)
+              : ex.nidx != nullptr          ? form(ke->f16_2d, ke->bf16_2d)
+              : sorts                       ? form(ke->f16_sort, ke->bf16_sort)
+                                            : form(ke->f16, ke->bf16);
   if (topk && (fn == nullptr || (mode == MODE_TOPK_SELF && pl.rows_per_group != 16)))
     return fail(BSG_ERR_UNSUPPORTED, "top-k in the GEMM: no selection instantiation for this tile (kinds 1, 2, 4-7; "
                 "self-scored: fp16, 16-row tiles)");
