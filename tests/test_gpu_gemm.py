@@ -713,3 +713,41 @@ def test_plans_by_size(dev, bt, k, n, na, dtype):
     assert np.array_equal(ids[:c].cpu().numpy(), kept)
     ref = orc.gemm_ref64(xo, wo, kept)
     assert np.linalg.norm(y.float().cpu().numpy() - ref) <= 2.0 ** -8 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("plan", [(1, 16, 1, 4, 16, 1), (2, 16, 4, 4, 16, 1), (1, 16, 4, 4, 16, 6), (1, 32, 8, 2, 64, 7)])
+@pytest.mark.parametrize("nblk", [1, 31, 33, 64, 65, 512, 513, 1025, 2048])
+def test_lists_sorted_in_the_kernel_over_every_bitmap_word(dev, plan, nblk):
+    """The in-kernel sort at the edges of its bitmap (one word per 32 blocks, one lane per word) and of
+    its passes over the list (one per work-group's threads): the bits of the GEMM on the sorted list,
+    for distinct ids, and for lists with an equal or an out-of-range id (ranked instead)."""
+    n, bt = 48, 3 if plan[4] == 16 else 50
+    g = torch.Generator(device=dev).manual_seed(nblk)
+    # whole numbers whose sums fp32 holds exactly, so that no order of summation shows
+    x = torch.randint(-2, 3, (bt, 64 * nblk), generator=g, device=dev).half()
+    w = torch.randint(-1, 2, (n, 64 * nblk), generator=g, device=dev).half()
+    packed = bsa.pack_weight(w)
+    p = bsa.Plan(*plan)
+    rng = np.random.default_rng(nblk)
+    for na in sorted({a for a in (1, 2, 63, 64, 65, 256, 257, 512, 513, 1024, nblk) if a <= min(nblk, 1024)}):
+        perm = rng.permutation(nblk)[:na].astype(np.int32)
+        ends = perm.copy()
+        ends[:2] = [nblk - 1, 0][: ends[:2].size]  # the first and last bit, once each
+        lists = {"distinct": perm}
+        if np.unique(ends).size == na:
+            lists["ends"] = ends
+        if na > 1:
+            lists["equal"] = np.r_[perm[1:], perm[1:2]].astype(np.int32)
+            lists["past"] = np.r_[perm[:-1], nblk].astype(np.int32)
+            lists["negative"] = np.r_[-1, perm[1:]].astype(np.int32)
+        for what, ids in lists.items():
+            print(f"bitmap sort plan={plan} nblk={nblk} na={na} {what}", flush=True)
+            got = torch.full((bt, n), float("nan"), dtype=F16, device=dev)
+            want = got.clone()
+            bsa.gemm_packed(x, packed, n, to_dev(ids, dev), got, plan=p, sort_list=True)
+            bsa.gemm_packed(x, packed, n, to_dev(np.sort(ids), dev), want, plan=p)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (na, what)
+            real = torch.from_numpy(ids[(ids >= 0) & (ids < nblk)].astype(np.int64)).to(dev)
+            ch = (real[:, None] * 64 + torch.arange(64, device=dev)).reshape(-1)
+            ref = x[:, ch].double() @ w[:, ch].double().t()
+            assert torch.equal(got, ref.half()), (na, what)

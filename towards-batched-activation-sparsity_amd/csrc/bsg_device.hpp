@@ -513,13 +513,14 @@ __device__ __forceinline__ void tile_of_group(int split_k, int* tile, int* sk) {
 }
 
 // Distinct ids of [0, universe) (at most BSG_MAX_NBLK) in ascending order, handed to emit(position,
-// id): the ids set bits of an LDS bitmap, and each set bit's position is the count of set bits below
-// it.  `first` is ids[threadIdx.x], loaded by the caller ahead of whatever it waits for.  Returns
-// false, before any emit, when an id is out of range or occurs twice.  s_bm holds BSG_MAX_NBLK / 32
-// words that emit does not touch; the emitted values are unfenced.  Three dependent LDS steps whatever
-// the length, where ranking every entry against the list takes one LDS read per entry: a q/k/v/o
-// launch at 2 rows on 13 unsorted entries 4.58 -> 4.19 us, down at 16 rows on 86 entries (an eager
-// call) 14.3 -> 12.1.
+// id): the ids set bits of an LDS bitmap, and each id's position is the count of set bits below its
+// own.  `first` is ids[threadIdx.x] (0 past the list), loaded by the caller ahead of whatever it waits
+// for.  Returns false, before any emit, when an id is out of range or occurs twice.  s_bm holds
+// BSG_MAX_NBLK / 32 words, one per lane, that emit does not touch; the emitted values are unfenced.
+// Three barriers' worth of LDS steps and one pass over the list per NT entries, whatever the universe
+// (each wave scans the words' counts in registers), where ranking every entry against the list takes
+// one LDS read per entry (kind 6, 16 columns, 13 / 64 of 64 blocks 4.39 / 7.91 us ranked, 3.93 / 6.36
+// here, of 2048 blocks 4.47 / 8.07, 4.00 / 6.52); a list refused here pays both (4.38, 4.41 of 64).
 template <int NT, typename Emit>
 __device__ __forceinline__ bool sort_by_bitmap(const int32_t* ids, int n, int universe, int first, uint32_t* s_bm,
                                                Emit emit) {
@@ -533,13 +534,23 @@ __device__ __forceinline__ bool sort_by_bitmap(const int32_t* ids, int n, int un
     odd |= (unsigned)id >= (unsigned)universe || (atomicOr(&s_bm[id >> 5], bit) & bit) != 0;
   }
   if (__syncthreads_or(odd)) return false;
-  for (int t = tid; t < universe; t += NT) {
-    const uint32_t w = s_bm[t >> 5], bit = 1u << (t & 31);
-    if (w & bit) {
-      int r = __popc(w & (bit - 1));
-      for (int k = 0; k < (t >> 5); ++k) r += __popc(s_bm[k]);
-      emit(r, t);
-    }
+  static_assert(BSG_MAX_NBLK == 32 * 64, "one bitmap word per lane");
+  const int lane = tid & 63;
+  const uint32_t word = s_bm[lane];
+  int below = __popc(word);
+  below += __builtin_amdgcn_update_dpp(0, below, 0x111, 0xf, 0xf, true);
+  below += __builtin_amdgcn_update_dpp(0, below, 0x112, 0xf, 0xf, true);
+  below += __builtin_amdgcn_update_dpp(0, below, 0x114, 0xf, 0xf, true);
+  below += __builtin_amdgcn_update_dpp(0, below, 0x118, 0xf, 0xf, true);
+  const int r1 = __builtin_amdgcn_readlane(below, 15), r2 = r1 + __builtin_amdgcn_readlane(below, 31),
+            r3 = r2 + __builtin_amdgcn_readlane(below, 47);
+  below += (lane < 16 ? 0 : lane < 32 ? r1 : lane < 48 ? r2 : r3) - __popc(word);
+  for (int i0 = 0; i0 < n; i0 += NT) {  // all lanes stay in the shuffles
+    const int i = i0 + tid;
+    const int id = i0 == 0 ? first : i < n ? ids[i] : 0;
+    const int src = id >> 5;
+    const int r = __shfl(below, src, 64) + __popc((uint32_t)__shfl((int)word, src, 64) & ((1u << (id & 31)) - 1u));
+    if (i < n) emit(r, id);
   }
   return true;
 }
@@ -728,7 +739,7 @@ __device__ __forceinline__ void sort_block_list(const int32_t* ids, int na, int 
                          [&](int r, int id) { s_ids[r] = id; }))
     return;
   uint32_t* const s_key = (uint32_t*)s_ids;
-  for (int i = tid; i < na; i += NT) s_key[i] = (uint32_t)(0x7fffffffLL - (long long)ids[i]);
+  for (int i = tid; i < na; i += NT) s_key[i] = (uint32_t)(0x7fffffffLL - (long long)(i == tid ? first : ids[i]));
   __syncthreads();
   int* const s_out = s_ids + BSG_MAX_NBLK / 2;
   for (int i = tid; i < na; i += NT) {
