@@ -33,5 +33,8 @@ def test_pack_sources_bit_exact(dev, layout, n, k, lead, skip):
     view = wide[:, skip:skip + src.shape[1]]
     view.copy_(src)
     for w in (src, view, view.view(torch.bfloat16)):
+        # the packed tensor is likely to take the memory of this one, not the previous answer's
+        del_me = torch.full(want.shape, float("nan"), dtype=torch.float16, device=dev)
+        del del_me
         got = bsa.pack_weight(w, layout=layout).view(torch.float16).cpu().numpy()
         assert np.array_equal(got.view(np.uint16), want), (layout, n, k, tuple(w.stride()))

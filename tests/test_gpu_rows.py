@@ -43,11 +43,12 @@ def test_rows_kernel(dev, cols, bt, k, n):
     ref = orc.gemm_ref64(x, w_nk, np.arange(nblk))
     ids = np.repeat(np.arange(nblk), 2).astype(np.int32)
     ids[1::2] = np.where(np.arange(nblk) % 2, -1, nblk)
-    out = torch.empty_like(out)
+    # (every output starts as NaN: memory reused from the loop above may hold the right answer)
+    out = torch.full_like(out, float("nan"))
     cnt = torch.tensor([2 * nblk], dtype=torch.int32, device=dev)
     bsa.gemm_packed(xt, packed, n, to_dev(np.r_[ids, ids], dev), out, plan=p, num_active_dev=cnt)
     bit = torch.ones(nblk, dtype=torch.uint8, device=dev)
-    out_b, out_d = torch.empty_like(out), torch.empty_like(out)
+    out_b, out_d = torch.full_like(out, float("nan")), torch.full_like(out, float("nan"))
     bsa.gemm_packed(xt, packed, n, None, out_b, bitmap=bit, plan=p)
     bsa.gemm_packed(xt, packed, n, None, out_d, plan=p)
     for o in (out, out_b, out_d):
@@ -64,8 +65,9 @@ def test_rows_kernel_bf16_and_stale_slots(dev):
     xb, wb = torch.from_numpy(x).to(torch.bfloat16), torch.from_numpy(w_nk).to(torch.bfloat16)
     packed = bsa.pack_weight(wb.to(dev))
     every = torch.arange(orc.nblk_of(k), dtype=torch.int32, device=dev)
-    out = torch.empty(bt, n, dtype=torch.bfloat16, device=dev)
+    out = torch.full((bt, n), float("nan"), dtype=torch.bfloat16, device=dev)
     bsa.gemm_packed(torch.full((bt, k), float("inf"), dtype=torch.bfloat16, device=dev), packed, n, every, out, plan=p)
+    out.fill_(float("nan"))
     bsa.gemm_packed(xb.to(dev), packed, n, to_dev(idx, dev), out, plan=p)
     ref = orc.gemm_ref64(xb.float().numpy(), wb.float().numpy(), idx)
     got = out.float().cpu().numpy()
@@ -80,11 +82,12 @@ def test_many_rows_through_the_public_calls(dev, bt, k, n, na):
     entry (which keeps its own tiles)."""
     x, w_nk, idx = case(bt, bt, k, n, na, "normal")
     xt, wt = to_dev(x, dev).view(bt, 1, k), to_dev(w_nk, dev)
-    out = torch.empty(bt, 1, n, dtype=torch.float16, device=dev)
+    out = torch.full((bt, 1, n), float("nan"), dtype=torch.float16, device=dev)
     bsa._prepacked_block_sparse_gemm_from_active_blocks(xt, wt, to_dev(idx[::-1].copy(), dev), out, cache_prefix="rows")
     assert_close(out.view(bt, n).float().cpu().numpy(), orc.gemm_ref64(x, w_nk, idx), "drop-in")
     want = tuning.many_rows_plan(bt, n)
     assert bsa.resolve_plan(bt, n, orc.nblk_of(k), na, dev).as_tuple() == want.as_tuple()
+    out.fill_(float("nan"))
     sel, _ = bsa.select_sparse_gemm(xt, wt, out, na, cache_prefix="rows")
     kept = sel.cpu().numpy()
     assert np.array_equal(kept, orc.select_topk_l1(x, na))
