@@ -80,18 +80,19 @@ enum bsg_status {
  *        contiguous bytes per load) and read back in MFMA order instead of loaded into
  *        registers; the registers this frees allow four block-slice waves at 64 rows.
  *        split_k must be 1.
- *   Kind 8 is for batches of more than 64 rows and refused below: 128-row groups x column groups
- *   dealt as in kind 5, both operands of every block loaded once into an LDS ring that all waves
- *   share (waves_per_group / 2 row parts x the two channel halves); waves_per_group 8, depth (ring
- *   stages) 4, split_k 1; no in-GEMM selection (a selection call runs a rank launch instead).
+ *     8  for batches of more than 64 rows, refused below: 128-row groups x column groups dealt as in
+ *        kind 5, both operands of every block loaded once into an LDS ring that all waves share
+ *        (waves_per_group / 2 row parts x the two channel halves).  waves_per_group 8, depth (ring
+ *        stages) 4, split_k must be 1; no in-GEMM selection (a selection call runs a rank launch
+ *        instead).
  *   Kinds 5-8 run 1-D lists only (bsg_gemm_2d rejects them), and only the tiles compiled
  *   into the library resolve (BSG_ERR_UNSUPPORTED names any other); a zero field of a kind 5-8
  *   plan takes rows 16/32/64 from bt (kind 8: 128), cols_per_wave 48, waves_per_group 4 (kind 8: 8),
  *   depth 4.
  * kind 0 here resolves by heuristic to kind 1 (bt <= 16) or kind 2 (larger bt).  The Python
  * layer does not rely on it: its plans come from a table tuned on the MI355X
- * (bsa_mi355x/tuned_plans.json) whose entries name kinds 1, 2, 4, 5, 6 and 7, or from
- * first-call tuning of problems the table does not hold.
+ * (bsa_mi355x/tuned_plans.json) whose entries name kinds 1, 2, 4, 5, 6 and 7, from first-call
+ * tuning of problems the table does not hold, or by size (more than 64 rows: kinds 4, 7 and 8).
  * Maps onto the reference's Triton tile (BLOCK_B, BLOCK_N, num_warps, num_stages) and
  * split-K factor (shared_mask_batched_triton_min_runtime.py:1296-1299, 1350-1361). */
 typedef struct bsg_plan {

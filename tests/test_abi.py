@@ -119,7 +119,7 @@ def _accepted_kinds():
     counts with every other field left automatic."""
     out = set()
     for kind in range(0, 10):
-        for bt, rows in ((16, 16), (64, 64), (32, 32), (4, 4)):
+        for bt, rows in ((16, 16), (64, 64), (32, 32), (4, 4), (128, 128)):
             if _resolve(bt, 4096, 64, 32, plan=_lib.Plan(0, 0, 0, 0, rows, kind))[0] == 0:
                 out.add(kind)
                 break
@@ -132,10 +132,10 @@ def test_header_documents_every_plan_kind():
     table names is among them (a C caller reading the header can form any shipped plan)."""
     doc = _plan_doc_kinds()
     accepted = _accepted_kinds() - {0}
-    assert accepted == {1, 2, 3, 4, 5, 6, 7}
+    assert accepted == {1, 2, 3, 4, 5, 6, 7, 8}
     assert set(doc) == accepted, (sorted(doc), sorted(accepted))
     for kind in accepted:
-        rows = 4 if kind == 3 else 16
+        rows = 4 if kind == 3 else 128 if kind == 8 else 16
         rc_sk2 = _resolve(rows, 4096, 64, 32, plan=_lib.Plan(2, 0, 0, 0, rows, kind))[0]
         single = "split_k must be 1" in doc[kind]
         assert (rc_sk2 == _lib.BSG_ERR_UNSUPPORTED) == single, (kind, rc_sk2, doc[kind])
