@@ -852,20 +852,12 @@ __device__ __forceinline__ void store_y(const GemmParams& p, int y0, int n0, int
   if (b >= p.bt) return;
   uint16_t* yrow = (uint16_t*)p.y + (size_t)b * (size_t)p.ldy;
   // One 8-byte store of the lane's 4 columns, whatever the row's alignment (global stores need only
-  // their elements').  The last columns of an N that is not a multiple of 4 go one by one, behind a
-  // scalar branch: behind a lane's own the epilogue of every launch paid for them (fused gate/up 31
-  // blocks, 64 rows 20.88 us against 20.6, q/k/v 13 blocks, 32 rows 7.48 / 7.3).
-  const bool whole = n + 4 <= p.ny;
-  auto store4 = [&] {
+  // their elements'); the last columns of an N that is not a multiple of 4 go one by one.
+  if (n + 4 <= p.ny) {
     u32x2_a2 pk;
     pk.x = (uint32_t)Elem<T>::bits(v.x) | ((uint32_t)Elem<T>::bits(v.y) << 16);
     pk.y = (uint32_t)Elem<T>::bits(v.z) | ((uint32_t)Elem<T>::bits(v.w) << 16);
     *(u32x2_a2*)(yrow + n) = pk;
-  };
-  if ((p.ny & 3) == 0) {
-    if (whole) store4();
-  } else if (whole) {
-    store4();
   } else {
     if (n + 0 < p.ny) yrow[n + 0] = Elem<T>::bits(v.x);
     if (n + 1 < p.ny) yrow[n + 1] = Elem<T>::bits(v.y);
