@@ -556,7 +556,7 @@ __device__ __forceinline__ bool sort_by_bitmap(const int32_t* ids, int n, int un
 }
 
 // The bi-th lowest id of an unsorted output-block list, found by every work-group for itself (a
-// down call at 16 rows on 86 K-blocks and 32 output blocks: 11.1 us, 13.4 with both lists ranked
+// down call at 16 rows on 86 K-blocks and 32 output blocks: 10.4 us, 13.4 with both lists ranked
 // entry by entry, 39.5 with two sort launches in front): a bitmap of the ids, or, for a list with
 // equal or out-of-range ids, each entry ranked against the whole list (equal ids by position).
 template <int NT>
