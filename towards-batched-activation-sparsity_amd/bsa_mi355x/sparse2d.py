@@ -116,8 +116,9 @@ def gemm_2d_packed(x2d: torch.Tensor, packed: torch.Tensor, n_dim: int, active_b
     `num_n_dev`.  sort_active: the GEMM sorts the K-block list ascending itself (at most
     MAX_NBLK // 2 entries); n_sorted_out (int32, at least num_n): n_blocks is in any order (at most
     SORT_N_MAX entries) and the GEMM takes its num_n lowest, writing them there ascending, while the
-    lists are still read: memory of its own (both with host counts only).  compact=False: y2d is [bt, N] and only the active blocks' columns are
-    written; compact=True: y2d is [bt, num_n * 64], list entry i at columns 64i.."""
+    lists are still read: memory of its own (both with host counts only).  compact=False: y2d is
+    [bt, N] and only the active blocks' columns are written; compact=True: y2d is [bt, num_n * 64],
+    list entry i at columns 64i.."""
     lib = load()
     dev = _require_cuda(x2d, packed, y2d)
     code = _dtype_code(x2d)
