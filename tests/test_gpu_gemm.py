@@ -674,7 +674,9 @@ def test_variable_width_column_groups(dev, bt, k, n, na):
 
 @pytest.mark.parametrize("bt,k,n,na", [(1, 2048, 2048, 16), (16, 1000, 8200, 9), (24, 1024, 13824, 12),
                                        (33, 512, 20000, 8), (64, 640, 16384, 10), (48, 4096, 4096, 64),
-                                       (40, 8192, 4096, 100)])
+                                       (40, 8192, 4096, 100),
+                                       # few column tiles and a long list: split over the idle units
+                                       (1, 12288, 500, 190), (9, 8192, 1003, 110), (24, 8192, 520, 120)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_plans_by_size(dev, bt, k, n, na, dtype):
     """Shapes the table does not hold, under capture (no first-call tuning) and through a selection:

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 
 import bsa_mi355x as bsa  # noqa: E402
 from bsa_mi355x import tuning  # noqa: E402
+from bsa_mi355x.select import select_gemm_packed  # noqa: E402
 
 
 @pytest.mark.parametrize("cols", [32, 48, 64, 96])
@@ -100,3 +101,28 @@ def test_many_rows_through_the_public_calls(dev, bt, k, n, na):
     got = out.view(bt, n).float().cpu().numpy()
     assert_close(got[:, cols], orc.gemm_ref64(x, w_nk, idx)[:, cols], "2-D")
     assert not np.delete(got, cols, axis=1).any()
+
+
+@pytest.mark.parametrize("bt,k,n,na,select_kind", [
+    (160, 4096, 4096, 64, 4),    # kind 4 over a long list: split two ways, three row groups
+    (320, 4160, 2050, 50, 4),    # split three ways, five row groups, odd width of the last subtile
+    (72, 1024, 11016, 12, 7),    # a GEMM on kind 8, a selection on kind 7
+    (128, 4096, 6912, 31, 7),    # four subtiles per unit on kind 7
+    (320, 1024, 8200, 9, 8),     # kind 8 over two rounds of 64 columns
+])
+def test_many_rows_plans_by_list_length_and_selection(dev, bt, k, n, na, select_kind):
+    """The automatic plans past 64 rows that depend on the list's length or on a selection."""
+    nblk = orc.nblk_of(k)
+    x, w_nk, idx = case(bt, bt, k, n, na, "normal")
+    xt, packed = to_dev(x, dev), bsa.pack_weight(to_dev(w_nk, dev))
+    pl = tuning.many_rows_plan(bt, n, na)
+    out = torch.full((bt, n), float("nan"), dtype=torch.float16, device=dev)
+    print(f"many rows bt={bt} K={k} N={n} na={na} plan={pl.as_tuple()}", flush=True)
+    bsa.gemm_packed(xt, packed, n, to_dev(idx, dev), out, plan=pl)
+    assert_close(out.float().cpu().numpy(), orc.gemm_ref64(x, w_nk, idx), "list")
+    assert bsa.resolve_plan(bt, n, nblk, na, dev, select=True).kind == select_kind
+    out.fill_(float("nan"))
+    sel, _ = select_gemm_packed(xt, packed, n, na, out)
+    kept = sel.cpu().numpy()
+    assert np.array_equal(kept, orc.select_topk_l1(x, na))
+    assert_close(out.float().cpu().numpy(), orc.gemm_ref64(x, w_nk, kept), "selection")
